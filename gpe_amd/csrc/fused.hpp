@@ -45,8 +45,8 @@ struct PairInfo {
 };
 
 template <typename T, int R, int NW, int P, int D, int PAIR, bool COMP>
-__device__ __forceinline__ void pair_tile(const StageArgs &A, const StageArgs &B, const int tx, const int ty,
-                                          const int z0, const int z1, const int slot, double *pn, double *pe) {
+__device__ __forceinline__ void pair_tile(const StageArgs &A, const StageArgs &B, const int tx, const int ty, const int z0,
+                                          const int z1, const int slot, double *pn, double *pe) {
   using PI = PairInfo<PAIR>;
   constexpr int KA = PI::KA, KB = PI::KB;
   constexpr int TX = 64, TY = NW * P, TXO = TX - 2 * R, TYO = TY - 2 * R;
@@ -215,9 +215,9 @@ __device__ __forceinline__ void pair_tile(const StageArgs &A, const StageArgs &B
   // ... and the k_A terms added when k_A is known (last in each sum)
   auto finish_F = [&](cx<T> *F, cx<T> ka) {
     if constexpr (KB == K_RK4_2) {
-      F[0] = rdiv(ka, B.d6, 1.0 / 6.0);
+      F[0] = rdiv(ka, div_of(B.d6), 1.0 / 6.0);
     } else if constexpr (KB == K_RK4_4) {
-      F[1] = F[1] + rdiv(ka, B.d3, 1.0 / 3.0);
+      F[1] = F[1] + rdiv(ka, div_of(B.d3), 1.0 / 3.0);
     } else if constexpr (KB == K_CK_6) {
       if constexpr (COMP) {
         F[2] = axpy<COMP>((T)ck_dc(5), ka, F[2]);
@@ -363,12 +363,12 @@ __device__ __forceinline__ void pair_tile(const StageArgs &A, const StageArgs &B
         ym2 = LD(-2 * LXA);
         yp2 = LD(2 * LXA);
       }
-      const cx<T> dxx = d2<T, R>(xm2, xm1, c0, xp1, xp2, A.d_xx, A.inv_xx);
-      const cx<T> dyy = d2<T, R>(ym2, ym1, c0, yp1, yp2, A.d_yy, A.inv_yy);
-      const cx<T> dzz = d2<T, R>(qA[0][p], qA[R - 1][p], c0, qA[R + 1][p], qA[2 * R][p], A.d_zz, A.inv_zz);
+      const cx<T> dxx = d2<T, R>(xm2, xm1, c0, xp1, xp2, div_of(A.d_xx), A.inv_xx);
+      const cx<T> dyy = d2<T, R>(ym2, ym1, c0, yp1, yp2, div_of(A.d_yy), A.inv_yy);
+      const cx<T> dzz = d2<T, R>(qA[0][p], qA[R - 1][p], c0, qA[R + 1][p], qA[2 * R][p], div_of(A.d_zz), A.inv_zz);
       const cx<T> lap = (dxx + dyy) + dzz;
       cx<T> dpx = mk((T)0, (T)0);
-      if (A.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, A.d_x, A.inv_x);
+      if (A.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, div_of(A.d_x), A.inv_x);
       const cx<T> f = rhs_site<T>(A, c0, lap, dpx, gim, gjm[p], kam);
       cx<T> kA;
       if constexpr (PI::is_ck) {
@@ -451,12 +451,12 @@ __device__ __forceinline__ void pair_tile(const StageArgs &A, const StageArgs &B
           ym2 = LY(0);
           yp2 = LY(3);
         }
-        const cx<T> dxx = d2<T, R>(xm2, xm1, c0, xp1, xp2, B.d_xx, B.inv_xx);
-        const cx<T> dyy = d2<T, R>(ym2, ym1, c0, yp1, yp2, B.d_yy, B.inv_yy);
-        const cx<T> dzz = d2<T, R>(qB[0][p], qB[R - 1][p], c0, qB[R + 1][p], qB[2 * R][p], B.d_zz, B.inv_zz);
+        const cx<T> dxx = d2<T, R>(xm2, xm1, c0, xp1, xp2, div_of(B.d_xx), B.inv_xx);
+        const cx<T> dyy = d2<T, R>(ym2, ym1, c0, yp1, yp2, div_of(B.d_yy), B.inv_yy);
+        const cx<T> dzz = d2<T, R>(qB[0][p], qB[R - 1][p], c0, qB[R + 1][p], qB[2 * R][p], div_of(B.d_zz), B.inv_zz);
         const cx<T> lap = (dxx + dyy) + dzz;
         cx<T> dpx = mk((T)0, (T)0);
-        if (B.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, B.d_x, B.inv_x);
+        if (B.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, div_of(B.d_x), B.inv_x);
         const cx<T> f = rhs_site<T>(B, c0, lap, dpx, gi, gj[p], k);
         const size_t s = (size_t)k * plane + (size_t)gj[p] * nx + gi;
         cx<T> F[NFA];
@@ -464,10 +464,10 @@ __device__ __forceinline__ void pair_tile(const StageArgs &A, const StageArgs &B
         for (int q = 0; q < NFA; ++q) F[q] = FF[0][p][q];
         if constexpr (KB == K_RK4_2) {
           stc<T>(B.kout, s, f);
-          stc<T>(B.acc_out, s, F[0] + rdiv(f, B.d3, 1.0 / 3.0));
+          stc<T>(B.acc_out, s, F[0] + rdiv(f, div_of(B.d3), 1.0 / 3.0));
         } else if constexpr (KB == K_RK4_4) {
           const cx<T> ps = F[0];
-          const cx<T> incr = F[1] + rdiv(f, B.d6, 1.0 / 6.0);
+          const cx<T> incr = F[1] + rdiv(f, div_of(B.d6), 1.0 / 6.0);
           cx<double> np;
           if constexpr (IS_DBL) {
             np = ps + cmul(mk((T)B.dtr, (T)B.dti), incr);

@@ -13,18 +13,6 @@
 #include "host_common.h"
 
 namespace gpe {
-// Division by a real constant in the reference's form (see stage_args.h).
-DivC make_divc(double s) {
-  DivC d{};
-  int e = ilogb(s);
-  d.e = e;
-  d.cs = ldexp(s, -e);
-  d.den = d.cs * d.cs + 0.0 * 0.0;
-  return d;
-}
-}  // namespace gpe
-
-namespace gpe {
 
 void fill_base(const gpe_params *params, int prec, StageArgs &A) {
   const int R = params->order / 2;

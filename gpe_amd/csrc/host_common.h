@@ -19,7 +19,6 @@ int fail(int code, const char *fmt, ...);
     if (e_ != hipSuccess) return ::gpe::fail(GPE_EHIP, "%s: %s", #call, hipGetErrorString(e_)); \
   } while (0)
 
-DivC make_divc(double s);
 // Geometry, coefficients and constant divisors of one simulation (no field
 // pointers, no dt).
 void fill_base(const gpe_params *params, int prec, StageArgs &A);

@@ -18,15 +18,9 @@ __global__ void __launch_bounds__(256) norm_kernel(const void *psi, const void *
   const size_t end = beg + chunk < n ? beg + chunk : n;
   double acc = 0.0;
   for (size_t s = beg + threadIdx.x; s < end; s += blockDim.x) {
-    double m2;
-    if constexpr (std::is_same<T, double>::value) {
-      double m = cabs_(ldc<double>(psi, s));
-      m2 = m * m;  // abs(in_var)**2
-    } else {
-      cx<double> v = todbl(ldc<T>(psi, s));
-      if constexpr (COMP) v = v + todbl(ldc<T>(lo, s));
-      m2 = v.re * v.re + v.im * v.im;
-    }
+    cx<double> v = todbl(ldc<T>(psi, s));
+    if constexpr (COMP) v = v + todbl(ldc<T>(lo, s));
+    double m2 = v.re * v.re + v.im * v.im;  // abs(in_var)**2
     if (weighted) {
       const int i = (int)(s % nx);
       const size_t r = s / nx;

@@ -45,8 +45,7 @@ namespace refm {
 // ax >= ay > 0, both in range: h = sqrt(ax^2 + ay^2), then the correction.
 // Both correction formulas are evaluated and one is selected (no divergent
 // branch on the device); each is the same expression either way.
-GPE_HD double hypot_kernel(double ax, double ay) {
-  const double h = std::sqrt(ax * ax + ay * ay);
+GPE_HD double hypot_sum(double ax, double ay, double h, double &two_h) {
   const bool near = h <= 2.0 * ay;
   const double d1 = h - ay, d2 = h - ax;
   const double t1a = ax * (2.0 * d1 - ax);
@@ -54,12 +53,48 @@ GPE_HD double hypot_kernel(double ax, double ay) {
   const double t1b = 2.0 * d2 * (ax - 2.0 * ay);
   const double t2b = (4.0 * d2 - ay) * ay + d2 * d2;
   const double t1 = near ? t1a : t1b, t2 = near ? t2a : t2b;
-  return h - (t1 + t2) / (2.0 * h);
+  two_h = 2.0 * h;
+  return t1 + t2;
 }
 
-// Operands out of the kernel's range: non-finite, very large or very small,
-// or so different in size that the smaller one does not count.
-GPE_HD double hypot_edge(double x, double y) {
+GPE_HD double hypot_kernel(double ax, double ay) {
+  const double h = std::sqrt(ax * ax + ay * ay);
+  double two_h;
+  const double n = hypot_sum(ax, ay, h, two_h);
+  return h - n / two_h;
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// The same for 2^-383 <= ax: the general FP64 sqrt and division spend 89 and
+// 71 cycles per wave on an MI355X (an FMA takes 5), much of it on scaling
+// for operands that do not occur in this range.  Here h and y = 1/(2h) come
+// from one reciprocal square root by Goldschmidt's iteration, h is rounded
+// by two residual corrections, and the quotient takes y after one Newton
+// step and a residual correction: 89 + 71 -> about 85 cycles, the same bits
+// (P. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", IBM J. Res. Dev. 34, 1990, for the corrections).
+__device__ __forceinline__ double hypot_fast(double ax, double ay) {
+  const double x = ax * ax + ay * ay;
+  double y = __builtin_amdgcn_rsq(x);
+  double g = x * y;
+  y = 0.5 * y;
+  const double r = __builtin_fma(-y, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  y = __builtin_fma(y, r, y);
+  g = __builtin_fma(__builtin_fma(-g, g, x), y, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), y, g);
+  double two_h;
+  const double n = hypot_sum(ax, ay, g, two_h);
+  y = __builtin_fma(y, __builtin_fma(-two_h, y, 1.0), y);
+  double q = n * y;
+  q = __builtin_fma(__builtin_fma(-two_h, q, n), y, q);
+  return g - q;
+}
+#endif
+
+// Every operand: scaled into the kernel's range where it is very large or
+// very small; the larger one alone where the smaller does not count.
+GPE_HD double hypot_any(double x, double y) {
   constexpr double kScale = 0x1p-600, kLarge = 0x1p+511, kTiny = 0x1p-511, kEps = 0x1p-54;
   if (!std::isfinite(x) || !std::isfinite(y)) {
     if (std::isinf(x) || std::isinf(y)) return INFINITY;
@@ -68,24 +103,32 @@ GPE_HD double hypot_edge(double x, double y) {
   x = std::fabs(x);
   y = std::fabs(y);
   const double ax = x < y ? y : x, ay = x < y ? x : y;
+  bool alone;
+  double in = 1.0, out = 1.0;
   if (ax > kLarge) {
-    if (ay <= ax * kEps) return ax + ay;
-    return hypot_kernel(ax * kScale, ay * kScale) / kScale;
+    alone = ay <= ax * kEps;
+    in = kScale;
+    out = 1.0 / kScale;
+  } else if (ay < kTiny) {
+    alone = ax >= ay / kEps;
+    in = 1.0 / kScale;
+    out = kScale;
+  } else {
+    alone = ay <= ax * kEps;
   }
-  if (ay < kTiny) {
-    if (ax >= ay / kEps) return ax + ay;
-    return hypot_kernel(ax / kScale, ay / kScale) * kScale;
-  }
-  return ax + ay;  // ay <= ax * kEps
+  if (alone) return ax + ay;
+  return hypot_kernel(ax * in, ay * in) * out;
 }
 
 GPE_HD double hypot_ref(double x, double y) {
-  constexpr double kLarge = 0x1p+511, kTiny = 0x1p-511, kEps = 0x1p-54;
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr double kLarge = 0x1p+511, kEps = 0x1p-54, kSmall = 0x1p-383;
   const double fx = std::fabs(x), fy = std::fabs(y);
   const double ax = fx < fy ? fy : fx, ay = fx < fy ? fx : fy;
-  // false for NaN and infinite operands, which take the edge path
-  if (ax <= kLarge && ay >= kTiny && ay > ax * kEps) return hypot_kernel(ax, ay);
-  return hypot_edge(x, y);
+  // false for NaN and infinite operands
+  if (ax <= kLarge && ax >= kSmall && ay > ax * kEps) return hypot_fast(ax, ay);
+#endif
+  return hypot_any(x, y);
 }
 
 // --- double-double arithmetic (Dekker 1971; Knuth TAOCP vol. 2, 4.2.2) -----

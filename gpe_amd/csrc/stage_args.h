@@ -6,6 +6,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "divc.h"
+
 namespace gpe {
 
 // One fused sweep of the time-stepping path.  Each kind reads psi and the
@@ -61,16 +63,6 @@ __host__ __device__ constexpr double ck_dc(int m) {
 
 // Two consecutive stages fused into one sweep (fused.hpp).
 enum Pair : int { P_RK4_12 = 0, P_RK4_34, P_CK_12, P_CK_34, P_CK_56, P_COUNT };
-
-// Division by a real constant as the reference build evaluates it: the
-// divisor is promoted to complex and divided by compiler-rt's logb-scaled
-// quotient, i.e. ((a*cs + b*0)/den, (b*cs - a*0)/den) * 2^-e with
-// cs = s*2^-e, den = cs*cs + 0*0, e = logb(s).
-struct DivC {
-  double cs, den;
-  int e;
-  int pad;
-};
 
 struct StageArgs {
   // geometry and tiling

@@ -38,6 +38,42 @@
 
 namespace gpe {
 
+// The launch descriptor of an FP64 tile, in uniform memory (the kernel
+// arguments, or an instance's entry of a batch table) that does not change
+// while the kernel runs.  Named by its address space, fresh() can have
+// members loaded again where they are used: the equations 1..3 have some 20
+// coefficients that an eqn-4 run never reads; kept over the whole march they
+// push the FP64 kernels' scalars into lanes of vector registers (11 to 69 per
+// kernel), each use costing an instruction.  (Loading every member again each
+// plane removes the rest of those, but its latency costs as much: FP64 512^3
+// step 13.3 ms against 13.0 ms.)  The FP32 kernels' scalars fit.
+using UniformArgs = const __attribute__((address_space(4))) StageArgs;
+
+__device__ __forceinline__ UniformArgs &fresh(UniformArgs &a) {
+  UniformArgs *p = &a;
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+__device__ __forceinline__ const StageArgs &fresh(const StageArgs &a) { return a; }
+
+template <typename T>
+using Args = typename std::conditional<std::is_same<T, double>::value, UniformArgs, const StageArgs>::type;
+
+// The descriptor at p (global memory) as a tile of T reads it.
+template <typename T>
+__device__ __forceinline__ Args<T> &args_at(const StageArgs *p) {
+  return *(Args<T> *)p;
+}
+
+__device__ __forceinline__ DivC div_of(const __attribute__((address_space(4))) DivC &d) {
+  DivC r;
+  r.cs = d.cs;
+  r.zh = d.zh;
+  r.zl = d.zl;
+  return r;
+}
+__device__ __forceinline__ DivC div_of(const DivC &d) { return d; }
+
 template <typename T>
 using vec2_t = typename std::conditional<std::is_same<T, double>::value, double2, float2>::type;
 
@@ -87,13 +123,15 @@ __device__ __forceinline__ void stc(void *p, size_t i, cx<T> a) {
 #endif
 }
 
-// complex / real constant
-__device__ __forceinline__ cx<double> rdiv(cx<double> a, const DivC &d, double) {
-  double x = (a.re * d.cs + a.im * 0.0) / d.den;
-  double y = (a.im * d.cs - a.re * 0.0) / d.den;
-  return mk(ldexp(x, -d.e), ldexp(y, -d.e));
+// complex / real constant (divc.h); the reference's + im*0 and - re*0 stay (a
+// non-finite part reaches the other): the product is exact, so the sum
+// rounds once as there
+__device__ __forceinline__ cx<double> rdiv(cx<double> a, DivC d, double) {
+  const double x = fma(a.im, 0.0, a.re * d.cs);
+  const double y = fma(-a.re, 0.0, a.im * d.cs);
+  return mk(div_const(x, d), div_const(y, d));
 }
-__device__ __forceinline__ cx<float> rdiv(cx<float> a, const DivC &, double inv) {
+__device__ __forceinline__ cx<float> rdiv(cx<float> a, DivC, double inv) {
   float f = (float)inv;
   return mk(a.re * f, a.im * f);
 }
@@ -166,6 +204,44 @@ __device__ __forceinline__ double err_ratio2(cx<float> e, cx<float> sc) {
   return fma(er, er, ei * ei) / fma(sr, sr, si * si);
 }
 
+// The rk45 error measure is a maximum over the grid, so |err/scale| itself
+// (two divisions and a hypot in FP64 and FP32, an FP64 division and two
+// square roots in the compensated form) is needed only where it can exceed
+// the largest value this wave has met: sites with |err|^2 <= thr * s2 (s2
+// at most |scale|^2) cannot, where thr is that largest value squared, taken
+// down by a margin far above the rounding of this test.  A wave meets a new
+// largest value about log(planes) times in a march, so nearly every site
+// takes the test alone: 7 operations.  Products outside the normal range
+// decide nothing, and NaN passes the test on, so the measure's value, NaN and
+// infinities are those of testing every site.
+__device__ __forceinline__ bool err_may_lead(cx<double> e, double s2, double thr) {
+  const double m2 = fma(e.re, e.re, e.im * e.im), t = thr * s2;
+  return !(m2 <= t && t >= 1e-280 && t <= 1e300);
+}
+__device__ __forceinline__ bool err_may_lead(cx<float> e, float s2, float thr) {
+  const float m2 = fmaf(e.re, e.re, e.im * e.im), t = thr * s2;
+  return !(m2 <= t && t >= 1e-36f && t <= 1e37f);
+}
+// The next thr of a wave whose lanes' largest values are m (NaN: ignored),
+// all lanes active.  A maximum over the lanes in single precision, by lane
+// shifts within the vector unit (rounding is inside the margin; a value
+// outside the single range gives a thr that decides nothing).
+template <typename T>
+__device__ __forceinline__ T err_lead(double m) {
+  float x = fmaxf((float)m, 0.0f);
+  auto shifted = [&](auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  x = fmaxf(x, shifted(std::integral_constant<int, 0x111>()));  // row_shr:1, 2, 4, 8
+  x = fmaxf(x, shifted(std::integral_constant<int, 0x112>()));
+  x = fmaxf(x, shifted(std::integral_constant<int, 0x114>()));
+  x = fmaxf(x, shifted(std::integral_constant<int, 0x118>()));
+  x = fmaxf(x, shifted(std::integral_constant<int, 0x142>()));  // row_bcast:15, 31
+  x = fmaxf(x, shifted(std::integral_constant<int, 0x143>()));
+  x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+  return (T)x * (T)x * (T)(1.0 - 0x1p-10);
+}
+
 // Index map for a ghost index i in [-R, n-1+R].
 __device__ __forceinline__ int bcmap(int i, int n, int periodic) {
   if (periodic) return i < 0 ? i + n : (i >= n ? i - n : i);
@@ -194,7 +270,7 @@ __device__ __forceinline__ double nweight(int i, int n, double w1, double w2, do
 // estimate (itself a ~1e-6 fraction of the stage values) above rounding
 // noise.
 template <typename T, int R>
-__device__ __forceinline__ cx<T> d2(cx<T> m2, cx<T> m1, cx<T> c, cx<T> p1, cx<T> p2, const DivC &d,
+__device__ __forceinline__ cx<T> d2(cx<T> m2, cx<T> m1, cx<T> c, cx<T> p1, cx<T> p2, DivC d,
                                     double inv) {
   if constexpr (std::is_same<T, double>::value) {
     if constexpr (R == 1) {
@@ -217,7 +293,7 @@ __device__ __forceinline__ cx<T> d2(cx<T> m2, cx<T> m1, cx<T> c, cx<T> p1, cx<T>
 
 // deriv_x (derivs.f90:41-57)
 template <typename T, int R>
-__device__ __forceinline__ cx<T> d1(cx<T> m2, cx<T> m1, cx<T> p1, cx<T> p2, const DivC &d, double inv) {
+__device__ __forceinline__ cx<T> d1(cx<T> m2, cx<T> m1, cx<T> p1, cx<T> p2, DivC d, double inv) {
   if constexpr (R == 1) {
     return rdiv(p1 - m1, d, inv);
   } else {
@@ -228,12 +304,13 @@ __device__ __forceinline__ cx<T> d1(cx<T> m2, cx<T> m1, cx<T> p1, cx<T> p2, cons
 
 // get_rhs at one site (solve.f90:414-437).
 template <typename T>
-__device__ __forceinline__ cx<T> rhs_site(const StageArgs &A, cx<T> u, cx<T> lap, cx<T> dpx, int i, int j,
+__device__ __forceinline__ cx<T> rhs_site(Args<T> &A0, cx<T> u, cx<T> lap, cx<T> dpx, int i, int j,
                                           int k) {
-  const T x = (T)A.xl + (T)i * (T)A.dx;
-  const T y = (T)A.yl + (T)j * (T)A.dy;
-  const T z = (T)A.zl + (T)k * (T)A.dz;
-  if (A.eqn == 4) {
+  if (A0.eqn == 4) {
+    Args<T> &A = A0;
+    const T x = (T)A.xl + (T)i * (T)A.dx;
+    const T y = (T)A.yl + (T)j * (T)A.dy;
+    const T z = (T)A.zl + (T)k * (T)A.dz;
     T V = (T)0.5 * (((T)A.ox2 * (x * x) + (T)A.oy2 * (y * y)) + (T)A.oz2 * (z * z));
     T s;
     if constexpr (std::is_same<T, double>::value) {
@@ -249,6 +326,10 @@ __device__ __forceinline__ cx<T> rhs_site(const StageArgs &A, cx<T> u, cx<T> lap
     cx<T> in = ((t1 + t2) + t3) - t4;
     return mk(in.im, -in.re);  // -eye*(...)
   }
+  Args<T> &A = fresh(A0);
+  const T x = (T)A.xl + (T)i * (T)A.dx;
+  const T y = (T)A.yl + (T)j * (T)A.dy;
+  const T z = (T)A.zl + (T)k * (T)A.dz;
   T m = cabs_(u);
   T m2 = m * m;
   cx<T> r;
@@ -295,7 +376,7 @@ struct FifoInfo {
   static constexpr int nf = KIND == K_RK2_2   ? 1   // psi
                             : KIND == K_RK4_2 ? 1   // kk1/6
                             : KIND == K_RK4_4 ? 2   // psi, acc + kk3/3
-                            : KIND == K_CK_6  ? (COMP ? 4 : 2)  // psi_hi, sum c kk, sum dc kk, scale | psi + sum c kk, sum dc kk
+                            : KIND == K_CK_6  ? (COMP ? 4 : 2)  // psi_hi, sum c kk, sum dc kk, kk1 | psi + sum c kk, sum dc kk
                                               : 0;
 };
 
@@ -333,7 +414,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // partial sums go to slot `slot` of the partial arrays pn / pe / pen (any
 // of them may be null).
 template <typename T, int R, int NW, int P, int KIND, bool COMP>
-__device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, const int ty, const int z0,
+__device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int ty, const int z0,
                                            const int z1, const int slot, double *pn, double *pe, double *pen) {
   constexpr int TX = 64, TY = NW * P, LX = TX + 2 * R, LY = TY + 2 * R;
   constexpr int NQ = 2 * R + 1;
@@ -441,10 +522,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
     if constexpr (KIND == K_RK2_2) {
       F[0] = r.ps;
     } else if constexpr (KIND == K_RK4_2) {
-      F[0] = rdiv(r.kk[0], A.d6, 1.0 / 6.0);  // kk1/6
+      F[0] = rdiv(r.kk[0], div_of(A.d6), 1.0 / 6.0);  // kk1/6
     } else if constexpr (KIND == K_RK4_4) {
       F[0] = r.ps;
-      F[1] = r.ac + rdiv(r.kk[0], A.d3, 1.0 / 3.0);  // (kk1/6 + kk2/3) + kk3/3
+      F[1] = r.ac + rdiv(r.kk[0], div_of(A.d3), 1.0 / 3.0);  // (kk1/6 + kk2/3) + kk3/3
     } else if constexpr (KIND == K_CK_6) {
       cx<T> pe = rmul((T)ck_dc(1), r.kk[0]);
 #pragma unroll
@@ -456,7 +537,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
         F[0] = r.ps;
         F[1] = pd;
         F[2] = pe;
-        F[3] = scale_from_kk1(A, r.ps, r.kk[0]);
+        F[3] = r.kk[0];
       } else {
         cx<T> pn = r.ps;
 #pragma unroll
@@ -552,6 +633,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
   issue_out(z0);
 
   double acc_norm = 0.0, acc_emax = 0.0, acc_en = 0.0;
+  T thr = (T)-1;  // err_may_lead: every site of the first plane is measured
 
   // one plane of the march; rb/hb hold plane k+R and are refilled with
   // plane k+D+R
@@ -612,9 +694,9 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
         yp2 = LD(2 * LX);
       }
       const cx<T> zm1 = q[R - 1][p], zp1 = q[R + 1][p];
-      const cx<T> dxx = d2<T, R>(xm2, xm1, c0, xp1, xp2, A.d_xx, A.inv_xx);
-      const cx<T> dyy = d2<T, R>(ym2, ym1, c0, yp1, yp2, A.d_yy, A.inv_yy);
-      const cx<T> dzz = d2<T, R>(zm2, zm1, c0, zp1, zp2, A.d_zz, A.inv_zz);
+      const cx<T> dxx = d2<T, R>(xm2, xm1, c0, xp1, xp2, div_of(A.d_xx), A.inv_xx);
+      const cx<T> dyy = d2<T, R>(ym2, ym1, c0, yp1, yp2, div_of(A.d_yy), A.inv_yy);
+      const cx<T> dzz = d2<T, R>(zm2, zm1, c0, zp1, zp2, div_of(A.d_zz), A.inv_zz);
       const cx<T> lap = (dxx + dyy) + dzz;
       const bool act = act_x && (gj[p] < ny);
       const size_t s = (size_t)k * plane + (size_t)gj[p] * nx + gi;
@@ -622,20 +704,27 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
       if constexpr (KIND == K_ENERGY) {
         if (act) {
           cx<T> pr = cmul(mk(-lap.re, -lap.im), mk(c0.re, -c0.im));
-          T m = cabs_(c0);
-          T m2 = m * m;
+          T m2;
+          if constexpr (IS_DBL) {
+            m2 = c0.re * c0.re + c0.im * c0.im;
+          } else {
+            const T m = cabs_(c0);
+            m2 = m * m;
+          }
           acc_en += (double)(pr.re + (T)0.5 * (m2 * m2));
         }
       } else {
         cx<T> dpx = mk((T)0, (T)0);
-        if (A.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, A.d_x, A.inv_x);
+        if (A.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, div_of(A.d_x), A.inv_x);
         const cx<T> f = rhs_site<T>(A, c0, lap, dpx, gi, gj[p], k);
+        cx<T> err = mk((T)0, (T)0);
+        bool lead = false;
         if (act) {
           if constexpr (KIND == K_RHS || KIND == K_RK2_1 || KIND == K_RK4_1 || KIND == K_RK4_3) {
             stc<T>(A.kout, s, f);
           } else if constexpr (KIND == K_RK4_2) {
             stc<T>(A.kout, s, f);
-            stc<T>(A.acc_out, s, F[0][p][0] + rdiv(f, A.d3, 1.0 / 3.0));
+            stc<T>(A.acc_out, s, F[0][p][0] + rdiv(f, div_of(A.d3), 1.0 / 3.0));
           } else if constexpr (KI::is_ck) {
             cx<T> kk;  // kk = dt*f
             if constexpr (IS_DBL || !COMP) {
@@ -662,40 +751,27 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
               stc<T>(A.kout, s, kk);
             } else {
               // K_CK_6: new state and the error norm (solve.f90:365-375, 184)
-              const cx<T> sc = COMP ? F[0][p][NF - 1] : oc[p][0];
-              const cx<T> err = F[0][p][COMP ? 2 : 1] + rmul((T)ck_dc(6), kk);
+              err = F[0][p][COMP ? 2 : 1] + rmul((T)ck_dc(6), kk);
               cx<double> np;
               if constexpr (IS_DBL) {
                 np = F[0][p][0] + rmul((T)ck_c(6), kk);
                 stc<T>(A.psi_out, s, np);
-                const double e = cabs_(cdiv(err, sc));
-                acc_emax = (e > acc_emax || e != e) ? e : acc_emax;
+              } else if constexpr (COMP) {
+                const cx<double> dl = todbl(F[0][p][1]) + rmul(ck_c(6), todbl(kk));
+                np = (todbl(F[0][p][0]) + todbl(oc[p][0])) + dl;
+                const cx<T> hi = mk((T)np.re, (T)np.im);
+                stc<T>(A.psi_out, s, hi);
+                stc<T>(A.lo_out, s, mk((T)(np.re - (double)hi.re), (T)(np.im - (double)hi.im)));
               } else {
-                if constexpr (COMP) {
-                  const cx<double> dl = todbl(F[0][p][1]) + rmul(ck_c(6), todbl(kk));
-                  np = (todbl(F[0][p][0]) + todbl(oc[p][0])) + dl;
-                  const cx<T> hi = mk((T)np.re, (T)np.im);
-                  stc<T>(A.psi_out, s, hi);
-                  stc<T>(A.lo_out, s, mk((T)(np.re - (double)hi.re), (T)(np.im - (double)hi.im)));
-                  // |err/scale|^2, maximised; its square root after the march
-                  const double e2 = err_ratio2(err, sc);
-                  acc_emax = (e2 > acc_emax || e2 != e2) ? e2 : acc_emax;
-                } else {
-                  const cx<T> nf = F[0][p][0] + rmul((T)ck_c(6), kk);
-                  stc<T>(A.psi_out, s, nf);
-                  np = todbl(nf);
-                  // abs(err/scale) (solve.f90:184) in single precision
-                  const float e = cabs_(cdiv(err, sc));
-                  acc_emax = ((double)e > acc_emax || e != e) ? (double)e : acc_emax;
-                }
+                const cx<T> nf = F[0][p][0] + rmul((T)ck_c(6), kk);
+                stc<T>(A.psi_out, s, nf);
+                np = todbl(nf);
               }
+              // |scale|^2, or in the compensated form its term |psi|^2
+              const cx<T> sc = COMP ? F[0][p][0] : oc[p][0];
+              lead = err_may_lead(err, sc.re * sc.re + sc.im * sc.im, thr);
               const double wn = wx * wy[p] * nweight(k, nz, A.w1, A.w2, A.w3);
-              if constexpr (IS_DBL) {
-                const double mm = cabs_(np);
-                acc_norm += wn * (mm * mm);
-              } else {
-                acc_norm += wn * (np.re * np.re + np.im * np.im);
-              }
+              acc_norm += wn * (np.re * np.re + np.im * np.im);
             }
           } else if constexpr (KI::final_) {
             // K_EULER, K_RK2_2, K_RK4_4
@@ -708,7 +784,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
               incr = f;
             } else {
               ps = F[0][p][0];
-              incr = F[0][p][1] + rdiv(f, A.d6, 1.0 / 6.0);
+              incr = F[0][p][1] + rdiv(f, div_of(A.d6), 1.0 / 6.0);
             }
             cx<double> np;
             if constexpr (IS_DBL) {
@@ -725,12 +801,23 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
               np = todbl(nf);
             }
             const double wn = wx * wy[p] * nweight(k, nz, A.w1, A.w2, A.w3);
-            if constexpr (IS_DBL) {
-              const double mm = cabs_(np);
-              acc_norm += wn * (mm * mm);
-            } else {
-              acc_norm += wn * (np.re * np.re + np.im * np.im);
+            acc_norm += wn * (np.re * np.re + np.im * np.im);
+          }
+        }
+        if constexpr (KIND == K_CK_6) {
+          if (__any(lead)) {
+            if (lead) {
+              if constexpr (COMP) {
+                // |err/scale|^2, maximised; its square root after the march
+                const double e2 = err_ratio2(err, scale_from_kk1(A, F[0][p][0], F[0][p][NF - 1]));
+                acc_emax = (e2 > acc_emax || e2 != e2) ? e2 : acc_emax;
+              } else {
+                // abs(err/scale) (solve.f90:184), in the storage precision
+                const T e = cabs_(cdiv(err, oc[p][0]));
+                acc_emax = ((double)e > acc_emax || e != e) ? (double)e : acc_emax;
+              }
             }
+            thr = err_lead<T>(COMP ? sqrt(acc_emax) : acc_emax);
           }
         }
       }
@@ -795,9 +882,19 @@ __device__ __forceinline__ void stage_tile(const StageArgs &A, const int tx, con
   }
 }
 
+// The kernel's only argument, as a tile of T reads it.
+template <typename T>
+__device__ __forceinline__ Args<T> &only_argument(const StageArgs &D) {
+  if constexpr (std::is_same<T, double>::value)
+    return *(UniformArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  else
+    return D;
+}
+
 // Single simulation: one workgroup per tile.
 template <typename T, int R, int NW, int P, int KIND, bool COMP>
-__global__ void __launch_bounds__(64 * NW) stage_kernel(const StageArgs A) {
+__global__ void __launch_bounds__(64 * NW) stage_kernel(const StageArgs D) {
+  Args<T> &A = only_argument<T>(D);
   // XCD-aware tile order: the hardware deals consecutive workgroups round
   // robin over the 8 XCDs; give each XCD a contiguous range of tiles so
   // neighbouring tiles (which share ghost rows) run on one L2.
@@ -828,7 +925,7 @@ __global__ void __launch_bounds__(64 * NW)
   for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
     const WorkItem it = work[w];
     if (active[it.inst])
-      stage_tile<T, R, NW, P, KIND, COMP>(insts[it.inst], it.tx, it.ty, it.z0, it.z1, it.slot, pn, pe, nullptr);
+      stage_tile<T, R, NW, P, KIND, COMP>(args_at<T>(insts + it.inst), it.tx, it.ty, it.z0, it.z1, it.slot, pn, pe, nullptr);
     __syncthreads();  // the next item reuses the LDS tile
   }
 }
