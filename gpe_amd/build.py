@@ -54,6 +54,11 @@ for _v in range(N_VARIANTS):
     # into different kernels) compute bitwise the same field
     UNITS.append(("gpe_stage.hip", "stage_f32_v%d" % _v, ["-ffp-contract=off", "-DGPE_VID=%d" % _v, "-DGPE_NT_STORE"]))
 
+# brick sweeps: the next stage reads their outputs back from L2 or the
+# Infinity Cache, so they are stored plainly
+UNITS.append(("gpe_brick.hip", "brick_f64", ["-ffp-contract=off", "-DGPE_F64"]))
+UNITS.append(("gpe_brick.hip", "brick_f32", ["-ffp-contract=off"]))
+
 # fused stage pairs: FP32 forms only (three tile variants)
 for _v in range(3):
     UNITS.append(("gpe_pair.hip", "pair_f32_v%d" % _v, ["-ffp-contract=off", "-DGPE_PVID=%d" % _v, "-DGPE_NT_STORE"]))

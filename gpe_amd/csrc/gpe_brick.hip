@@ -1,0 +1,67 @@
+// gpe_brick.hip -- the brick sweeps (brick.hpp) of one precision, built like
+// the stage kernels of gpe_stage.hip.
+#include "brick.hpp"
+#include "launch.h"
+
+#ifdef GPE_F64
+#define GPE_REAL double
+#define GPE_BRICK launch_brick_f64
+#else
+#define GPE_REAL float
+#define GPE_BRICK launch_brick_f32
+#endif
+
+namespace gpe {
+
+namespace {
+template <int R, int KIND, bool COMP>
+hipError_t launch_one(int planes, const StageArgs &A, hipStream_t s) {
+#ifdef GPE_F64
+  // bricks of 4 planes: only the kinds brick_planes gives them to
+  if constexpr (stage_reads(KIND) <= 2 && KIND != K_ENERGY)
+    if (planes == 4) {
+      hipLaunchKernelGGL((brick_kernel<GPE_REAL, R, kBrickWaves, 4, KIND, COMP>), dim3(A.nblocks),
+                         dim3(64 * kBrickWaves), 0, s, A);
+      return hipGetLastError();
+    }
+#endif
+  if (planes != 2) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((brick_kernel<GPE_REAL, R, kBrickWaves, 2, KIND, COMP>), dim3(A.nblocks), dim3(64 * kBrickWaves),
+                     0, s, A);
+  return hipGetLastError();
+}
+
+template <int R, bool COMP>
+hipError_t launch_r(int planes, int kind, const StageArgs &A, hipStream_t s) {
+  switch (kind) {
+    case K_RHS: return launch_one<R, K_RHS, false>(planes, A, s);
+    case K_EULER: return launch_one<R, K_EULER, COMP>(planes, A, s);
+    case K_RK2_1: return launch_one<R, K_RK2_1, false>(planes, A, s);
+    case K_RK2_2: return launch_one<R, K_RK2_2, COMP>(planes, A, s);
+    case K_RK4_1: return launch_one<R, K_RK4_1, false>(planes, A, s);
+    case K_RK4_2: return launch_one<R, K_RK4_2, false>(planes, A, s);
+    case K_RK4_3: return launch_one<R, K_RK4_3, false>(planes, A, s);
+    case K_RK4_4: return launch_one<R, K_RK4_4, COMP>(planes, A, s);
+    case K_CK_1: return launch_one<R, K_CK_1, COMP>(planes, A, s);
+    case K_CK_2: return launch_one<R, K_CK_2, COMP>(planes, A, s);
+    case K_CK_3: return launch_one<R, K_CK_3, COMP>(planes, A, s);
+    case K_CK_4: return launch_one<R, K_CK_4, COMP>(planes, A, s);
+    case K_CK_5: return launch_one<R, K_CK_5, COMP>(planes, A, s);
+    case K_CK_6: return launch_one<R, K_CK_6, COMP>(planes, A, s);
+    case K_ENERGY: return launch_one<R, K_ENERGY, false>(planes, A, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+}  // namespace
+
+hipError_t GPE_BRICK(int planes, int kind, int radius, bool comp, const StageArgs &A, hipStream_t s) {
+#ifdef GPE_F64
+  (void)comp;
+  return radius == 1 ? launch_r<1, false>(planes, kind, A, s) : launch_r<2, false>(planes, kind, A, s);
+#else
+  if (radius == 1) return comp ? launch_r<1, true>(planes, kind, A, s) : launch_r<1, false>(planes, kind, A, s);
+  return comp ? launch_r<2, true>(planes, kind, A, s) : launch_r<2, false>(planes, kind, A, s);
+#endif
+}
+
+}  // namespace gpe

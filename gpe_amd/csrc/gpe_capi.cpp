@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
 #include <cfloat>
 #include <cmath>
@@ -107,8 +108,12 @@ struct gpe_ctx {
   // reductions
   double *part = nullptr;  // 3 * part_cap
   int part_cap = 0;
-  double *dscal = nullptr;   // device scalars: norm, emax, energy
-  double *hscal = nullptr;   // pinned mirror
+  double *hscal = nullptr;   // host memory the device writes: norm, emax, energy, ticket
+  double ticket = 0.0;       // of the last reduction into hscal
+  // norm history: partials of several steps, reduced together
+  double *hpart = nullptr;
+  int hsteps = 0, hpend = 0, hblocks = 0;  // steps hpart holds, pending ones, workgroups of each
+  double *hnext = nullptr;                 // where the first pending norm goes
   double *hist = nullptr;
   int64_t hist_cap = 0, hist_len = 0;
   bool uploaded = false;
@@ -146,6 +151,14 @@ struct gpe_ctx {
 namespace {
 
 int grid_for_v(gpe_ctx *c, int vid, int zc, StageArgs &A) { return stage_grid(c->P.nx, c->P.ny, c->P.nz, vid, zc, A); }
+
+// Planes per brick of a kind's sweep, 0 for the z march: bricks are the
+// automatic configuration's choice (default tile, automatic z-chunk) only.
+int bricks_of(const gpe_ctx *c, int kind) {
+  const bool fp64 = c->prec == GPE_FP64;
+  if (c->zc[kind] != 0 || c->vid[kind] != default_vid(fp64, kind)) return 0;
+  return brick_planes(fp64, kind, c->P.nx, c->P.ny, c->P.nz);
+}
 
 int grid_for(gpe_ctx *c, int kind, StageArgs &A) { return grid_for_v(c, c->vid[kind], c->zc[kind], A); }
 
@@ -197,15 +210,21 @@ void prof_drain(gpe_ctx *c) {
 
 int run_kind(gpe_ctx *c, int kind, StageArgs &A) {
   Range range(kind_name(kind));
-  grid_for(c, kind, A);
-  if (A.nblocks > c->part_cap) return fail(GPE_EINVAL, "internal: %d workgroups exceed partial buffer", A.nblocks);
+  const int bricks = bricks_of(c, kind);
+  if (bricks)
+    brick_grid(c->P.nx, c->P.ny, c->P.nz, bricks, A);
+  else
+    grid_for(c, kind, A);
+  if ((kind_final(kind) || kind == K_ENERGY) && A.nblocks > c->part_cap)
+    return fail(GPE_EINVAL, "internal: %d workgroups exceed partial buffer", A.nblocks);
   hipEvent_t ea = nullptr, eb = nullptr;
   if (c->prof) {
     ea = take_event(c);
     eb = take_event(c);
     if (ea) (void)hipEventRecord(ea, c->stream);
   }
-  hipError_t e = launch_stage((int)c->esz, c->vid[kind], kind, c->R, c->comp, A, c->stream);
+  hipError_t e = bricks ? launch_brick((int)c->esz, bricks, kind, c->R, c->comp, A, c->stream)
+                        : launch_stage((int)c->esz, c->vid[kind], kind, c->R, c->comp, A, c->stream);
   if (e != hipSuccess) return fail(GPE_EHIP, "stage %s launch: %s", kind_name(kind), hipGetErrorString(e));
   if (c->prof && ea && eb) {
     (void)hipEventRecord(eb, c->stream);
@@ -250,17 +269,73 @@ StageArgs args_for(gpe_ctx *c) {
   A.hr = 0.5 * c->st.dt_re;
   A.hi = 0.5 * c->st.dt_im;
   A.inv_absdt = 1.0 / std::hypot(c->st.dt_re, c->st.dt_im);
-  A.part_norm = c->part;
+  A.part_norm = c->hpart ? c->hpart + (size_t)c->hpend * c->part_cap : c->part;
   A.part_emax = c->part + c->part_cap;
   A.part_energy = c->part + 2 * c->part_cap;
   return A;
 }
 
-int reduce_after(gpe_ctx *c, const StageArgs &A, bool emax, bool energy, double *hist_slot) {
+// Reduce a sweep's n partials into hscal; scalars() waits for them.
+int reduce_scalars(gpe_ctx *c, const double *pn, const double *pe, const double *pen, int n, double *hist_slot) {
   const double dv = c->P.dx * c->P.dy * c->P.dz;
-  hipError_t e = launch_reduce(A.part_norm, emax ? A.part_emax : nullptr, energy ? A.part_energy : nullptr,
-                               A.nblocks, dv, c->P.eps, dv, c->dscal, hist_slot, c->stream);
+  c->ticket += 1.0;
+  hipError_t e = launch_reduce(pn, pe, pen, n, dv, c->P.eps, dv, c->hscal, hist_slot, c->ticket, c->stream);
   if (e != hipSuccess) return fail(GPE_EHIP, "reduce launch: %s", hipGetErrorString(e));
+  return GPE_OK;
+}
+
+// The scalars of the last reduction.  The host watches for the ticket the
+// kernel writes behind them (copying 24 bytes out and waiting for the stream
+// takes 14 us, as long as two sweeps of a 48^3 grid); a longer wait than 2 ms is
+// left to the stream.
+int scalars(gpe_ctx *c) {
+  auto here = [&] {
+    double got;
+    __atomic_load(c->hscal + 3, &got, __ATOMIC_ACQUIRE);
+    return got == c->ticket;
+  };
+  const auto limit = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+  do {
+    for (int i = 0; i < 64; ++i) {
+      if (here()) return GPE_OK;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() < limit);
+  HIPCHK(hipStreamSynchronize(c->stream));
+  return here() ? GPE_OK : fail(GPE_EHIP, "a reduction ended without its result");
+}
+
+// Norms of the steps whose partials are pending, into the history.
+int flush_norms(gpe_ctx *c) {
+  if (!c->hpend) return GPE_OK;
+  const int steps = c->hpend;
+  c->hpend = 0;
+  hipError_t e = launch_reduce_norms(c->hpart, c->part_cap, c->hblocks, steps, c->P.dx * c->P.dy * c->P.dz, c->hnext,
+                                     c->stream);
+  if (e != hipSuccess) return fail(GPE_EHIP, "reduce launch: %s", hipGetErrorString(e));
+  return GPE_OK;
+}
+
+// The norm of a fixed step's new state, where its history is kept (nobody
+// reads it otherwise): its partials wait in hpart until several steps are
+// reduced by one launch (one launch each takes 4.5 us, a sixth of a 64^3 step).
+int keep_norm(gpe_ctx *c, const StageArgs &A, double *hist_slot) {
+  if (!hist_slot) return GPE_OK;
+  if (!c->hpend) c->hnext = hist_slot;
+  c->hblocks = A.nblocks;
+  return ++c->hpend == c->hsteps ? flush_norms(c) : GPE_OK;
+}
+
+// Memory for the partials of several steps (8 MB at most, 64 steps at most,
+// one step at least), kept with the context.
+int norm_room(gpe_ctx *c) {
+  if (c->hpart) return GPE_OK;
+  const int steps = (int)std::max<int64_t>(1, std::min<int64_t>(64, (int64_t)1048576 / c->part_cap));
+  if (hipMalloc((void **)&c->hpart, sizeof(double) * (size_t)steps * c->part_cap) != hipSuccess) {
+    c->hpart = nullptr;
+    return fail(GPE_ENOMEM, "norm history partials");
+  }
+  c->hsteps = steps;
   return GPE_OK;
 }
 
@@ -280,7 +355,7 @@ int step_once(gpe_ctx *c, double *hist_slot) {
     A.psi_out = c->psi2;
     A.lo_out = c->lo2;
     if ((rc = run_kind(c, K_EULER, A))) return rc;
-    if ((rc = reduce_after(c, A, false, false, hist_slot))) return rc;
+    if ((rc = keep_norm(c, A, hist_slot))) return rc;
     swap_state(c);
   } else if (sch == GPE_RK2) {
     StageArgs A = args_for(c);
@@ -294,7 +369,7 @@ int step_once(gpe_ctx *c, double *hist_slot) {
     A.psi_out = c->psi2;
     A.lo_out = c->lo2;
     if ((rc = run_kind(c, K_RK2_2, A))) return rc;
-    if ((rc = reduce_after(c, A, false, false, hist_slot))) return rc;
+    if ((rc = keep_norm(c, A, hist_slot))) return rc;
     swap_state(c);
   } else if (sch == GPE_RK4 && c->fuse) {
     // stages (1,2) and (3,4) pairwise: fused, k1 and k3 never leave the sweep
@@ -316,7 +391,7 @@ int step_once(gpe_ctx *c, double *hist_slot) {
     A4.psi_out = c->psi2;
     A4.lo_out = c->lo2;
     if ((rc = run_two(c, P_RK4_34, A3, A4))) return rc;
-    if ((rc = reduce_after(c, A4, false, false, hist_slot))) return rc;
+    if ((rc = keep_norm(c, A4, hist_slot))) return rc;
     swap_state(c);
   } else if (sch == GPE_RK4) {
     // k[0]: k1 then k3 (k1 is folded into acc by stage 2), k[1]: k2
@@ -343,7 +418,7 @@ int step_once(gpe_ctx *c, double *hist_slot) {
     A.psi_out = c->psi2;
     A.lo_out = c->lo2;
     if ((rc = run_kind(c, K_RK4_4, A))) return rc;
-    if ((rc = reduce_after(c, A, false, false, hist_slot))) return rc;
+    if ((rc = keep_norm(c, A, hist_slot))) return rc;
     swap_state(c);
   } else {
     return GPE_EINVAL;  // rk45 is driven by step_rk45
@@ -407,17 +482,16 @@ int rkqs(gpe_ctx *c, double *hist_slot) {
       for (int s = 1; s <= 5; s += 2) {
         StageArgs A = ck_args(s), B = ck_args(s + 1);
         if ((rc = run_two(c, P_CK_12 + s / 2, A, B))) return rc;
-        if (s == 5 && (rc = reduce_after(c, B, true, false, hist_slot))) return rc;
+        if (s == 5 && (rc = reduce_scalars(c, B.part_norm, B.part_emax, nullptr, B.nblocks, hist_slot))) return rc;
       }
     } else {
       for (int s = 1; s <= 6; ++s) {
         StageArgs A = ck_args(s);
         if ((rc = run_kind(c, K_CK_1 + s - 1, A))) return rc;
-        if (s == 6 && (rc = reduce_after(c, A, true, false, hist_slot))) return rc;
+        if (s == 6 && (rc = reduce_scalars(c, A.part_norm, A.part_emax, nullptr, A.nblocks, hist_slot))) return rc;
       }
     }
-    HIPCHK(hipMemcpyAsync(c->hscal, c->dscal, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if ((rc = scalars(c))) return rc;
     const double em = c->hscal[1];  // maxval(|err/psi_scal|)/eps
     errmax = (RT)em;
     if (!(errmax == errmax)) return fail(GPE_ENONFINITE, "rk45: NaN in the error norm (t=%g)", c->st.t);
@@ -465,7 +539,7 @@ int solver_call(gpe_ctx *c, double *hist_slot) {
 
 void free_all(gpe_ctx *c) {
   void *ptrs[] = {c->psi, c->psi2, c->lo, c->lo2, c->k[0], c->k[1], c->k[2], c->k[3], c->k[4], c->k[5],
-                  c->acc, c->scale, c->part, c->dscal, c->hist, c->ll_buf, c->zr_buf, c->spec, c->spec_aux};
+                  c->acc, c->scale, c->part, c->hpart, c->hist, c->ll_buf, c->zr_buf, c->spec, c->spec_aux};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->hscal) (void)hipHostFree(c->hscal);
@@ -552,7 +626,7 @@ int gpe_ctx_create(const gpe_params *params, gpe_ctx **out) {
     // default launch configuration; partial buffers sized for the largest
     // grid any variant and z-chunk can produce
     for (int kk = 0; kk < K_COUNT; ++kk) {
-      c->vid[kk] = variant_allowed(c->prec == GPE_FP64, kk, kDefaultVid) ? kDefaultVid : kVidF64Ck;
+      c->vid[kk] = default_vid(c->prec == GPE_FP64, kk);
       c->zc[kk] = 0;
     }
     // every pair runs as its two stages until the autotuner (or
@@ -578,17 +652,22 @@ int gpe_ctx_create(const gpe_params *params, gpe_ctx **out) {
       int nb = grid_for_pair_v(c, v, 8, tmp);
       if (nb > cap) cap = nb;
     }
+    for (int kk = 0; kk < K_COUNT; ++kk) {
+      StageArgs tmp{};
+      const int b = kind_final(kk) || kk == K_ENERGY ? bricks_of(c, kk) : 0;
+      if (b) cap = std::max(cap, brick_grid(c->P.nx, c->P.ny, c->P.nz, b, tmp));
+    }
     if (cap < PW_BLOCKS) cap = PW_BLOCKS;
     c->part_cap = cap;
     if (hipMalloc((void **)&c->part, 3 * sizeof(double) * (size_t)cap) != hipSuccess) {
       rc = fail(GPE_ENOMEM, "partials");
       goto bad;
     }
-    if (hipMalloc((void **)&c->dscal, 4 * sizeof(double)) != hipSuccess ||
-        hipHostMalloc((void **)&c->hscal, 4 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void **)&c->hscal, 4 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
       rc = fail(GPE_ENOMEM, "scalars");
       goto bad;
     }
+    c->hscal[3] = 0.0;
   }
   fill_base(params, c->prec, c->base);
   *out = c;
@@ -648,14 +727,20 @@ int gpe_sim_advance(gpe_ctx *c, int64_t nsteps, int32_t record_norm) {
       c->hist_cap = nsteps;
     }
     c->hist_len = 0;
+    if (c->P.scheme != GPE_RK45)
+      if (int rc = norm_room(c)) return rc;
   }
   for (int64_t s = 0; s < nsteps; ++s) {
     double *slot = record_norm ? c->hist + s : nullptr;
     int rc = solver_call(c, slot);
-    if (rc) return rc;
+    if (rc) {
+      (void)flush_norms(c);
+      return rc;
+    }
     c->st.p += 1;
     if (record_norm) c->hist_len = s + 1;
   }
+  if (int rc = flush_norms(c)) return rc;
   if (c->prof) prof_drain(c);
   HIPCHK(hipStreamSynchronize(c->stream));
   return GPE_OK;
@@ -680,11 +765,8 @@ static int norm_like(gpe_ctx *c, int weighted, double *out) {
     e = launch_norm_f32(c->psi, c->comp ? c->lo : nullptr, A.nx, A.ny, A.nz, weighted, A.w1, A.w2, A.w3, c->part,
                         c->stream);
   if (e != hipSuccess) return fail(GPE_EHIP, "norm launch: %s", hipGetErrorString(e));
-  const double dv = c->P.dx * c->P.dy * c->P.dz;
-  e = launch_reduce(c->part, nullptr, nullptr, PW_BLOCKS, dv, c->P.eps, dv, c->dscal, nullptr, c->stream);
-  if (e != hipSuccess) return fail(GPE_EHIP, "reduce launch: %s", hipGetErrorString(e));
-  HIPCHK(hipMemcpyAsync(c->hscal, c->dscal, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  if (int rc = reduce_scalars(c, c->part, nullptr, nullptr, PW_BLOCKS, nullptr)) return rc;
+  if (int rc = scalars(c)) return rc;
   *out = c->hscal[0];
   return GPE_OK;
 }
@@ -699,9 +781,7 @@ int gpe_sim_energy(gpe_ctx *c, double *energy) {
   A.psi = c->psi;
   int rc = run_kind(c, K_ENERGY, A);
   if (rc) return rc;
-  if ((rc = reduce_after(c, A, false, true, nullptr))) return rc;
-  HIPCHK(hipMemcpyAsync(c->hscal, c->dscal, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  if ((rc = reduce_scalars(c, nullptr, nullptr, A.part_energy, A.nblocks, nullptr)) || (rc = scalars(c))) return rc;
   *energy = c->hscal[2];
   return GPE_OK;
 }

@@ -116,10 +116,80 @@ hipError_t launch_zeros(int prec, const void *psi, const void *lo, int nx, int n
   return hipGetLastError();
 }
 
+namespace {
+
+// Sum / max of a sweep's partials in a fixed order by one workgroup; thread 0
+// gets the results.
+constexpr int kReduceThreads = 256;
+__device__ __forceinline__ void reduce_all(const double *pn, const double *pe, const double *pen, int n, double &sum,
+                                           double &top, double &energy) {
+  __shared__ double s0[kReduceThreads], s1[kReduceThreads], s2[kReduceThreads];
+  double a = 0.0, m = 0.0, c = 0.0;
+  for (int i = threadIdx.x; i < n; i += kReduceThreads) {
+    if (pn) a += pn[i];
+    if (pe) m = (pe[i] > m || pe[i] != pe[i]) ? pe[i] : m;
+    if (pen) c += pen[i];
+  }
+  s0[threadIdx.x] = a;
+  s1[threadIdx.x] = m;
+  s2[threadIdx.x] = c;
+  __syncthreads();
+  for (int w = kReduceThreads / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) {
+      s0[threadIdx.x] += s0[threadIdx.x + w];
+      const double o = s1[threadIdx.x + w];
+      s1[threadIdx.x] = (o > s1[threadIdx.x] || o != o) ? o : s1[threadIdx.x];
+      s2[threadIdx.x] += s2[threadIdx.x + w];
+    }
+    __syncthreads();
+  }
+  sum = s0[0];
+  top = s1[0];
+  energy = s2[0];
+}
+
+// out[0] = sum(pn) * scale_norm, out[1] = max(pe) / eps (maxval(...)/eps,
+// solve.f90:184), out[2] = sum(pen) * scale_energy; hist (if set) gets out[0].
+// out may be host memory: with ticket != 0 the host reads out[0..2] once
+// out[3] holds the ticket, without a copy or a wait for the stream.
+__global__ void __launch_bounds__(kReduceThreads)
+    reduce_partials(const double *pn, const double *pe, const double *pen, int n, double scale_norm, double eps,
+                    double scale_energy, double *out, double *hist, double ticket) {
+  double a, m, c;
+  reduce_all(pn, pe, pen, n, a, m, c);
+  if (threadIdx.x == 0) {
+    out[0] = a * scale_norm;
+    out[1] = m / eps;
+    out[2] = c * scale_energy;
+    if (hist) *hist = a * scale_norm;
+    if (ticket != 0.0) {
+      __threadfence_system();
+      __hip_atomic_store(out + 3, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+}
+
+// The norms of several steps, one workgroup each: step b's partials start at
+// pn + b*stride.
+__global__ void __launch_bounds__(kReduceThreads)
+    reduce_norms(const double *pn, size_t stride, int n, double scale_norm, double *hist) {
+  double a, m, c;
+  reduce_all(pn + blockIdx.x * stride, nullptr, nullptr, n, a, m, c);
+  if (threadIdx.x == 0) hist[blockIdx.x] = a * scale_norm;
+}
+
+}  // namespace
+
 hipError_t launch_reduce(const double *pn, const double *pe, const double *pen, int n, double scale_norm,
-                         double eps, double scale_energy, double *out, double *hist, hipStream_t s) {
-  hipLaunchKernelGGL(reduce_partials, dim3(1), dim3(256), 0, s, pn, pe, pen, n, scale_norm, eps, scale_energy,
-                     out, hist);
+                         double eps, double scale_energy, double *out, double *hist, double ticket, hipStream_t s) {
+  hipLaunchKernelGGL(reduce_partials, dim3(1), dim3(kReduceThreads), 0, s, pn, pe, pen, n, scale_norm, eps,
+                     scale_energy, out, hist, ticket);
+  return hipGetLastError();
+}
+
+hipError_t launch_reduce_norms(const double *pn, size_t stride, int n, int steps, double scale_norm, double *hist,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(reduce_norms, dim3(steps), dim3(kReduceThreads), 0, s, pn, stride, n, scale_norm, hist);
   return hipGetLastError();
 }
 

@@ -68,7 +68,9 @@ extern "C" int gpe_energy_noalloc(const gpe_params *params, const void *psi, dou
   // the launch configuration of a new context (gpe_ctx_create), so the
   // partial sums and their order equal gpe_sim_energy's
   const int vid = kDefaultVid;
-  const int nb = stage_grid(params->nx, params->ny, params->nz, vid, 0, A);
+  const int bricks = brick_planes(prec == GPE_FP64, K_ENERGY, params->nx, params->ny, params->nz);
+  const int nb = bricks ? brick_grid(params->nx, params->ny, params->nz, bricks, A)
+                        : stage_grid(params->nx, params->ny, params->nz, vid, 0, A);
   if (nb > kMaxPartials)
     return fail(GPE_EINVAL, "grid %dx%dx%d needs %d workgroups; the no-allocation scratch holds %d partial sums",
                 params->nx, params->ny, params->nz, nb, kMaxPartials);
@@ -79,10 +81,13 @@ extern "C" int gpe_energy_noalloc(const gpe_params *params, const void *psi, dou
   A.part_norm = nullptr;
   A.part_emax = nullptr;
   A.part_energy = sp;
-  hipError_t e = launch_stage(prec == GPE_FP64 ? 16 : 8, vid, K_ENERGY, params->order / 2, prec == GPE_FP32C, A, s);
+  const int pb = prec == GPE_FP64 ? 16 : 8;
+  const bool comp = prec == GPE_FP32C;
+  hipError_t e = bricks ? launch_brick(pb, bricks, K_ENERGY, params->order / 2, comp, A, s)
+                        : launch_stage(pb, vid, K_ENERGY, params->order / 2, comp, A, s);
   if (e != hipSuccess) return fail(GPE_EHIP, "energy launch: %s", hipGetErrorString(e));
   const double dv = params->dx * params->dy * params->dz;
-  e = launch_reduce(nullptr, nullptr, sp, nb, dv, params->eps, dv, sp + kOut, nullptr, s);
+  e = launch_reduce(nullptr, nullptr, sp, nb, dv, params->eps, dv, sp + kOut, nullptr, 0.0, s);
   if (e != hipSuccess) return fail(GPE_EHIP, "reduce launch: %s", hipGetErrorString(e));
   e = hipMemcpyAsync(energy, sp + kOut + 2, sizeof(double), hipMemcpyDeviceToDevice, s);
   if (e != hipSuccess) return fail(GPE_EHIP, "result copy: %s", hipGetErrorString(e));

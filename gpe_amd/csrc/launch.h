@@ -32,6 +32,9 @@ constexpr bool variant_allowed(bool fp64, int kind, int vid) {
 
 // Tile variant of a new context's stage kinds (the (8,2) tile), where allowed.
 constexpr int kDefaultVid = 1;
+constexpr int default_vid(bool fp64, int kind) {
+  return variant_allowed(fp64, kind, kDefaultVid) ? kDefaultVid : kVidF64Ck;
+}
 
 // Tiling of one stage sweep over an nx x ny x nz grid with tile variant vid
 // and z-chunk zc (0: automatic): sets A.ntx, A.nty, A.zc, A.nzc and
@@ -57,6 +60,55 @@ inline int stage_grid(int nx, int ny, int nz, int vid, int zc, StageArgs &A) {
   A.nzc = (nz + zc - 1) / zc;
   A.nblocks = tiles2d * A.nzc;
   return A.nblocks;
+}
+
+// Fields a stage kind reads per site of its sweep.
+constexpr int stage_reads(int kind) {
+  return kind == K_RK2_2 || kind == K_RK4_2 || kind == K_RK4_3 ? 2
+         : kind == K_RK4_4                                     ? 3
+         : kind >= K_CK_1 && kind <= K_CK_6                    ? kind - K_CK_1 + 1
+                                                               : 1;
+}
+
+// Brick sweeps (brick.hpp): kBrickWaves rows and 2 or 4 planes per workgroup.
+constexpr int kBrickWaves = 8;
+inline int brick_grid(int nx, int ny, int nz, int planes, StageArgs &A) {
+  A.ntx = (nx + 63) / 64;
+  A.nty = (ny + kBrickWaves - 1) / kBrickWaves;
+  A.zc = planes;
+  A.nzc = (nz + planes - 1) / planes;
+  A.nblocks = A.ntx * A.nty * A.nzc;
+  return A.nblocks;
+}
+
+// Planes per brick with which a kind in its automatic configuration (default
+// tile, automatic z-chunk) sweeps a grid, or 0 for the z march.  A brick reads
+// each of its fields about three times (2 planes, 4th order) where the march
+// reads them once, so it pays while the march's chain of planes takes longer
+// than that: up to some number of field values per sweep, more in FP32, whose
+// values are half the size.  Measured (MI355X, us per sweep, march / 2 planes):
+//   FP64 4th order, ck_1: 48^3 22 / 8, 64^3 23 / 12, 128^3 47 / 35
+//   ck_3: 64^3 19 / 10, 96^3 35 / 24, 128^3 42 / 43
+//   ck_6: 64^3 32 / 15, 96^3 59 / 60, 128^3 72 / 129
+//   FP32C ck_6: 64^3 32 / 12, 96^3 35 / 29, 128^3 43 / 47; ck_3: 128^3 20.5 / 20.6
+// The FP64 kinds that read one field, or two on all but the largest grids,
+// take bricks of 4 planes beyond that: at 256^3 rk4_1 185 -> 135, rk4_2
+// 256 -> 231 (2nd order), ck_1 323 -> 206, ck_2 256 -> 226; at 384^3 rk4_1
+// 615 -> 425, but rk4_2 782 -> 866.
+inline int brick_planes(bool fp64, int kind, int nx, int ny, int nz) {
+  const long long n = (long long)nx * ny * nz;
+  const int reads = stage_reads(kind);
+  StageArgs A;
+  if (n * reads <= (fp64 ? 5000000 : 8000000)) return brick_grid(nx, ny, nz, 2, A) <= 65536 ? 2 : 0;
+  if (fp64 && kind != K_ENERGY && (reads == 1 || (reads == 2 && n <= 20000000))) return 4;
+  return 0;
+}
+hipError_t launch_brick_f64(int planes, int kind, int radius, bool comp, const StageArgs &A, hipStream_t s);
+hipError_t launch_brick_f32(int planes, int kind, int radius, bool comp, const StageArgs &A, hipStream_t s);
+inline hipError_t launch_brick(int prec_bytes, int planes, int kind, int radius, bool comp, const StageArgs &A,
+                               hipStream_t s) {
+  return prec_bytes == 16 ? launch_brick_f64(planes, kind, radius, comp, A, s)
+                          : launch_brick_f32(planes, kind, radius, comp, A, s);
 }
 
 // Launch stage kernel `kind` (radius 1 or 2) over A.nblocks workgroups with
@@ -109,9 +161,12 @@ hipError_t launch_pair_batched(int prec_bytes, int vid, int pair, int radius, bo
 hipError_t launch_batch_control(InstCtl *ctl, StageArgs *args, int cap, int *active, const int *range,
                                 const double *pn, const double *pe, hipStream_t s);
 
-// Reduce per-block partials to out[0..2] (see reduce_partials).
+// Reduce per-block partials to out[0..2], device memory or (ticket != 0) mapped
+// host memory (see reduce_partials); the norms of several steps at once.
 hipError_t launch_reduce(const double *pn, const double *pe, const double *pen, int n, double scale_norm,
-                         double eps, double scale_energy, double *out, double *hist, hipStream_t s);
+                         double eps, double scale_energy, double *out, double *hist, double ticket, hipStream_t s);
+hipError_t launch_reduce_norms(const double *pn, size_t stride, int n, int steps, double scale_norm, double *hist,
+                               hipStream_t s);
 
 // Pointwise helpers over a whole field.  Partials: one double per block.
 constexpr int PW_BLOCKS = 1024;

@@ -410,6 +410,276 @@ __device__ __forceinline__ void lds_barrier() { __syncthreads(); }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 #endif
 
+// Fields a stage reads at one site.
+template <typename T, int KIND>
+struct Raw {
+  cx<T> ps;
+  cx<T> kk[KindInfo<KIND>::nin > 0 ? KindInfo<KIND>::nin : 1];
+  cx<T> ac;
+};
+
+template <typename T, int KIND>
+__device__ __forceinline__ void load_raw(Args<T> &A, size_t s, Raw<T, KIND> &r, const bool full) {
+  constexpr int NIN = KindInfo<KIND>::nin;
+  r.ps = ldc<T>(A.psi, s);
+  if constexpr (NIN > 0) {
+#pragma unroll
+    for (int m = 0; m < NIN; ++m) r.kk[m] = ldc<T>(A.kin[m], s);
+  }
+  if constexpr (KindInfo<KIND>::has_acc) {
+    if (full) r.ac = ldc<T>(A.acc_in, s);
+  }
+}
+
+// stage input u = psi + sum coef * k (H: the RK2 and RK4 stages' coefficient)
+template <typename T, int KIND, bool COMP>
+__device__ __forceinline__ cx<T> stage_input(cx<T> H, const Raw<T, KIND> &r) {
+  constexpr int NIN = KindInfo<KIND>::nin;
+  if constexpr (NIN == 0) {
+    return r.ps;
+  } else if constexpr (KindInfo<KIND>::complex_coef) {
+    return r.ps + cmul(H, r.kk[0]);
+  } else {
+    cx<T> u = r.ps;
+#pragma unroll
+    for (int m = 0; m < NIN; ++m) u = axpy<COMP>((T)ck_b(KIND - K_CK_1 + 1, m), r.kk[m], u);
+    return u;
+  }
+}
+
+template <typename T, int KIND>
+__device__ __forceinline__ cx<T> stage_coef(Args<T> &A) {
+  return KIND == K_RK4_4 ? mk((T)A.dtr, (T)A.dti) : mk((T)A.hr, (T)A.hi);
+}
+
+// The pointwise terms of FifoInfo.
+template <typename T, int KIND, bool COMP>
+__device__ __forceinline__ void out_terms(Args<T> &A, const Raw<T, KIND> &r, cx<T> *F) {
+  if constexpr (KIND == K_RK2_2) {
+    F[0] = r.ps;
+  } else if constexpr (KIND == K_RK4_2) {
+    F[0] = rdiv(r.kk[0], div_of(A.d6), 1.0 / 6.0);  // kk1/6
+  } else if constexpr (KIND == K_RK4_4) {
+    F[0] = r.ps;
+    F[1] = r.ac + rdiv(r.kk[0], div_of(A.d3), 1.0 / 3.0);  // (kk1/6 + kk2/3) + kk3/3
+  } else if constexpr (KIND == K_CK_6) {
+    cx<T> pe = rmul((T)ck_dc(1), r.kk[0]);
+#pragma unroll
+    for (int m = 1; m < 5; ++m) pe = axpy<COMP>((T)ck_dc(m + 1), r.kk[m], pe);
+    if constexpr (COMP) {
+      cx<T> pd = rmul((T)ck_c(1), r.kk[0]);  // c2 = c5 = 0
+      pd = axpy<COMP>((T)ck_c(3), r.kk[2], pd);
+      pd = axpy<COMP>((T)ck_c(4), r.kk[3], pd);
+      F[0] = r.ps;
+      F[1] = pd;
+      F[2] = pe;
+      F[3] = r.kk[0];
+    } else {
+      cx<T> pn = r.ps;
+#pragma unroll
+      for (int m = 0; m < 5; ++m) pn = pn + rmul((T)ck_c(m + 1), r.kk[m]);
+      F[0] = pn;
+      F[1] = pe;
+    }
+  }
+}
+
+// The pointwise fields of OutInfo.
+template <typename T, int KIND, bool COMP>
+__device__ __forceinline__ void load_out(Args<T> &A, size_t s, cx<T> *o) {
+  int i = 0;
+  if constexpr (KIND == K_CK_6 && !COMP) {
+    // real time: the scale is real (its imaginary part is 0*|f|), stored as one word
+    if (A.scale_real)
+      o[i++] = mk(static_cast<const T *>(A.scale_in)[s], (T)0);
+    else
+      o[i++] = ldc<T>(A.scale_in, s);
+  }
+  if constexpr (COMP && KindInfo<KIND>::final_) {
+    // the low word is read at the tile's own sites only (no neighbour
+    // reads it as a ghost): stream it past L2
+    typedef T nv2 __attribute__((ext_vector_type(2)));
+    const nv2 v = __builtin_nontemporal_load(static_cast<const nv2 *>(A.lo) + s);
+    o[i++] = mk<T>(v.x, v.y);
+  }
+  (void)i;
+}
+
+// A thread's share of a sweep's reductions.
+template <typename T>
+struct Sums {
+  double norm = 0.0, emax = 0.0, en = 0.0;
+  T thr = (T)-1;  // err_may_lead: every site is measured until a wave has met one
+};
+
+// One site (i, j, k) at offset s: its right-hand side from the stage input c0,
+// its Laplacian and x-neighbours, and what the stage writes and sums there.
+// F: out_terms, o: load_out, wn: the site's get_norm weight.  All lanes of a
+// wave call it together (act: the lane's site is in the grid).
+template <typename T, int R, int KIND, bool COMP>
+__device__ __forceinline__ void emit_site(Args<T> &A, const bool act, const size_t s, const int i, const int j,
+                                          const int k, const cx<T> c0, const cx<T> lap, const cx<T> xm2,
+                                          const cx<T> xm1, const cx<T> xp1, const cx<T> xp2, const cx<T> *F,
+                                          const cx<T> *o, const double wn, Sums<T> &sum) {
+  using KI = KindInfo<KIND>;
+  constexpr bool IS_DBL = std::is_same<T, double>::value;
+  if constexpr (KIND == K_ENERGY) {
+    if (act) {
+      cx<T> pr = cmul(mk(-lap.re, -lap.im), mk(c0.re, -c0.im));
+      T m2;
+      if constexpr (IS_DBL) {
+        m2 = c0.re * c0.re + c0.im * c0.im;
+      } else {
+        const T m = cabs_(c0);
+        m2 = m * m;
+      }
+      sum.en += (double)(pr.re + (T)0.5 * (m2 * m2));
+    }
+  } else {
+    cx<T> dpx = mk((T)0, (T)0);
+    if (A.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, div_of(A.d_x), A.inv_x);
+    const cx<T> f = rhs_site<T>(A, c0, lap, dpx, i, j, k);
+    cx<T> err = mk((T)0, (T)0);
+    bool lead = false;
+    if (act) {
+      if constexpr (KIND == K_RHS || KIND == K_RK2_1 || KIND == K_RK4_1 || KIND == K_RK4_3) {
+        stc<T>(A.kout, s, f);
+      } else if constexpr (KIND == K_RK4_2) {
+        stc<T>(A.kout, s, f);
+        stc<T>(A.acc_out, s, F[0] + rdiv(f, div_of(A.d3), 1.0 / 3.0));
+      } else if constexpr (KI::is_ck) {
+        cx<T> kk;  // kk = dt*f
+        if constexpr (IS_DBL || !COMP) {
+          kk = cmul(mk((T)A.dtr, (T)A.dti), f);
+        } else {
+          // FP64 dt: no systematic bias from dt rounded to FP32
+          cx<double> kd = cmul(mk(A.dtr, A.dti), todbl(f));
+          kk = mk((T)kd.re, (T)kd.im);
+        }
+        if constexpr (KIND == K_CK_1) {
+          stc<T>(A.kout, s, kk);
+          if constexpr (!COMP) {
+            if (A.write_scale) {
+              // psi_scal = abs(in) + dt*abs(f) + 1e-30 (solve.f90:176-178)
+              T af = cabs_(f), au = cabs_(c0);
+              cx<T> sc = mk((au + (T)A.sdtr * af) + (T)1e-30, (T)A.sdti * af);
+              if (A.scale_real)
+                static_cast<T *>(A.scale_out)[s] = sc.re;
+              else
+                stc<T>(A.scale_out, s, sc);
+            }
+          }
+        } else if constexpr (KIND < K_CK_6) {
+          stc<T>(A.kout, s, kk);
+        } else {
+          // K_CK_6: new state and the error norm (solve.f90:365-375, 184)
+          err = F[COMP ? 2 : 1] + rmul((T)ck_dc(6), kk);
+          cx<double> np;
+          if constexpr (IS_DBL) {
+            np = F[0] + rmul((T)ck_c(6), kk);
+            stc<T>(A.psi_out, s, np);
+          } else if constexpr (COMP) {
+            const cx<double> dl = todbl(F[1]) + rmul(ck_c(6), todbl(kk));
+            np = (todbl(F[0]) + todbl(o[0])) + dl;
+            const cx<T> hi = mk((T)np.re, (T)np.im);
+            stc<T>(A.psi_out, s, hi);
+            stc<T>(A.lo_out, s, mk((T)(np.re - (double)hi.re), (T)(np.im - (double)hi.im)));
+          } else {
+            const cx<T> nf = F[0] + rmul((T)ck_c(6), kk);
+            stc<T>(A.psi_out, s, nf);
+            np = todbl(nf);
+          }
+          // |scale|^2, or in the compensated form its term |psi|^2
+          const cx<T> sc = COMP ? F[0] : o[0];
+          lead = err_may_lead(err, sc.re * sc.re + sc.im * sc.im, sum.thr);
+          sum.norm += wn * (np.re * np.re + np.im * np.im);
+        }
+      } else if constexpr (KI::final_) {
+        // K_EULER, K_RK2_2, K_RK4_4
+        cx<T> ps, incr;  // psi' = ps + dt*incr
+        if constexpr (KIND == K_EULER) {
+          ps = c0;
+          incr = f;
+        } else if constexpr (KIND == K_RK2_2) {
+          ps = F[0];
+          incr = f;
+        } else {
+          ps = F[0];
+          incr = F[1] + rdiv(f, div_of(A.d6), 1.0 / 6.0);
+        }
+        cx<double> np;
+        if constexpr (IS_DBL) {
+          np = ps + cmul(mk((T)A.dtr, (T)A.dti), incr);
+          stc<T>(A.psi_out, s, np);
+        } else if constexpr (COMP) {
+          np = (todbl(ps) + todbl(o[0])) + cmul(mk(A.dtr, A.dti), todbl(incr));
+          const cx<T> hi = mk((T)np.re, (T)np.im);
+          stc<T>(A.psi_out, s, hi);
+          stc<T>(A.lo_out, s, mk((T)(np.re - (double)hi.re), (T)(np.im - (double)hi.im)));
+        } else {
+          const cx<T> nf = ps + cmul(mk((T)A.dtr, (T)A.dti), incr);
+          stc<T>(A.psi_out, s, nf);
+          np = todbl(nf);
+        }
+        sum.norm += wn * (np.re * np.re + np.im * np.im);
+      }
+    }
+    if constexpr (KIND == K_CK_6) {
+      if (__any(lead)) {
+        if (lead) {
+          if constexpr (COMP) {
+            // |err/scale|^2, maximised; its square root after the march
+            const double e2 = err_ratio2(err, scale_from_kk1(A, F[0], F[3]));
+            sum.emax = (e2 > sum.emax || e2 != e2) ? e2 : sum.emax;
+          } else {
+            // abs(err/scale) (solve.f90:184), in the storage precision
+            const T e = cabs_(cdiv(err, o[0]));
+            sum.emax = ((double)e > sum.emax || e != e) ? (double)e : sum.emax;
+          }
+        }
+        sum.thr = err_lead<T>(COMP ? sqrt(sum.emax) : sum.emax);
+      }
+    }
+  }
+}
+
+// Deterministic block reductions: xor-shuffle within the wave, then the
+// waves in order, into slot `slot` of the partial arrays that are not null.
+template <typename T, int KIND, bool COMP, int NW>
+__device__ __forceinline__ void block_sums(Sums<T> &sum, double (*red)[NW], const int slot, double *pn, double *pe,
+                                           double *pen) {
+  // The compensated form maximised |err/scale|^2: the maximum of |err/scale|
+  // is its square root (monotone; NaN stays NaN).
+  if constexpr (KIND == K_CK_6 && COMP) sum.emax = sqrt(sum.emax);
+  if constexpr (KindInfo<KIND>::final_ || KIND == K_ENERGY) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      sum.norm += __shfl_xor(sum.norm, o);
+      sum.en += __shfl_xor(sum.en, o);
+      double om = __shfl_xor(sum.emax, o);
+      sum.emax = (om > sum.emax || om != om) ? om : sum.emax;
+    }
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+      red[0][wave] = sum.norm;
+      red[1][wave] = sum.emax;
+      red[2][wave] = sum.en;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double sn = 0.0, se = 0.0, mx = 0.0;
+      for (int w = 0; w < NW; ++w) {
+        sn += red[0][w];
+        se += red[2][w];
+        mx = (red[1][w] > mx || red[1][w] != red[1][w]) ? red[1][w] : mx;
+      }
+      if (pn) pn[slot] = sn;
+      if (pe) pe[slot] = mx;
+      if (pen) pen[slot] = se;
+    }
+  }
+}
+
 // One tile (64 x TY columns, planes z0 .. z1-1) of one stage sweep.  The per-block
 // partial sums go to slot `slot` of the partial arrays pn / pe / pen (any
 // of them may be null).
@@ -421,7 +691,6 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
   constexpr int NT = 64 * NW;
   using KI = KindInfo<KIND>;
   constexpr int NIN = KI::nin;
-  constexpr int NINA = NIN > 0 ? NIN : 1;
   constexpr int NF = FifoInfo<KIND, COMP>::nf;
   constexpr int NFA = NF > 0 ? NF : 1;
   constexpr int NO = OutInfo<KIND, COMP>::no;
@@ -433,12 +702,6 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
 
   __shared__ V lds[2][LY * LX];
   __shared__ double red[3][NW];
-
-  struct Raw {
-    cx<T> ps;
-    cx<T> kk[NINA];
-    cx<T> ac;
-  };
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -487,84 +750,13 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
     }
   }
 
-  const cx<T> H = KIND == K_RK4_4 ? mk((T)A.dtr, (T)A.dti) : mk((T)A.hr, (T)A.hi);
+  const cx<T> H = stage_coef<T, KIND>(A);
   // get_norm weights of this thread's column and rows (constant over the
   // z march); the product wx*wy*wz is formed in the same order as before
   const double wx = nweight(gi, nx, A.w1, A.w2, A.w3);
   double wy[P];
 #pragma unroll
   for (int p = 0; p < P; ++p) wy[p] = nweight(gj[p], ny, A.w1, A.w2, A.w3);
-
-  auto load_raw = [&](size_t s, Raw &r, const bool full) {
-    r.ps = ldc<T>(A.psi, s);
-    if constexpr (NIN > 0) {
-#pragma unroll
-      for (int m = 0; m < NIN; ++m) r.kk[m] = ldc<T>(A.kin[m], s);
-    }
-    if constexpr (KI::has_acc) {
-      if (full) r.ac = ldc<T>(A.acc_in, s);
-    }
-  };
-  // stage input u = psi + sum coef * k
-  auto make_u = [&](const Raw &r) -> cx<T> {
-    if constexpr (NIN == 0) {
-      return r.ps;
-    } else if constexpr (KI::complex_coef) {
-      return r.ps + cmul(H, r.kk[0]);
-    } else {
-      cx<T> u = r.ps;
-#pragma unroll
-      for (int m = 0; m < NIN; ++m) u = axpy<COMP>((T)ck_b(KIND - K_CK_1 + 1, m), r.kk[m], u);
-      return u;
-    }
-  };
-  auto make_F = [&](const Raw &r, cx<T> *F) {
-    if constexpr (KIND == K_RK2_2) {
-      F[0] = r.ps;
-    } else if constexpr (KIND == K_RK4_2) {
-      F[0] = rdiv(r.kk[0], div_of(A.d6), 1.0 / 6.0);  // kk1/6
-    } else if constexpr (KIND == K_RK4_4) {
-      F[0] = r.ps;
-      F[1] = r.ac + rdiv(r.kk[0], div_of(A.d3), 1.0 / 3.0);  // (kk1/6 + kk2/3) + kk3/3
-    } else if constexpr (KIND == K_CK_6) {
-      cx<T> pe = rmul((T)ck_dc(1), r.kk[0]);
-#pragma unroll
-      for (int m = 1; m < 5; ++m) pe = axpy<COMP>((T)ck_dc(m + 1), r.kk[m], pe);
-      if constexpr (COMP) {
-        cx<T> pd = rmul((T)ck_c(1), r.kk[0]);  // c2 = c5 = 0
-        pd = axpy<COMP>((T)ck_c(3), r.kk[2], pd);
-        pd = axpy<COMP>((T)ck_c(4), r.kk[3], pd);
-        F[0] = r.ps;
-        F[1] = pd;
-        F[2] = pe;
-        F[3] = r.kk[0];
-      } else {
-        cx<T> pn = r.ps;
-#pragma unroll
-        for (int m = 0; m < 5; ++m) pn = pn + rmul((T)ck_c(m + 1), r.kk[m]);
-        F[0] = pn;
-        F[1] = pe;
-      }
-    }
-  };
-  auto load_out = [&](size_t s, cx<T> *o) {
-    int i = 0;
-    if constexpr (KIND == K_CK_6 && !COMP) {
-      // real time: the scale is real (its imaginary part is 0*|f|), stored as one word
-      if (A.scale_real)
-        o[i++] = mk(static_cast<const T *>(A.scale_in)[s], (T)0);
-      else
-        o[i++] = ldc<T>(A.scale_in, s);
-    }
-    if constexpr (COMP && KI::final_) {
-      // the low word is read at the tile's own sites only (no neighbour
-      // reads it as a ghost): stream it past L2
-      typedef T nv2 __attribute__((ext_vector_type(2)));
-      const nv2 v = __builtin_nontemporal_load(static_cast<const nv2 *>(A.lo) + s);
-      o[i++] = mk<T>(v.x, v.y);
-    }
-    (void)i;
-  };
 
   cx<T> q[NQ][P];
   cx<T> F[R + 1][P][NFA];
@@ -579,20 +771,20 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
     const size_t zoff = (size_t)bcmap(z0 - R + m, nz, per) * plane;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      Raw r;
-      load_raw(zoff + roff[p], r, m >= R);
-      q[m][p] = make_u(r);
+      Raw<T, KIND> r;
+      load_raw<T, KIND>(A, zoff + roff[p], r, m >= R);
+      q[m][p] = stage_input<T, KIND, COMP>(H, r);
       if constexpr (NF > 0) {
-        if (m >= R) make_F(r, F[m - R][p]);
+        if (m >= R) out_terms<T, KIND, COMP>(A, r, F[m - R][p]);
       }
     }
     if (m >= R) {
 #pragma unroll
       for (int i = 0; i < HPT; ++i) {
         if (hl[i] >= 0) {
-          Raw r;
-          load_raw(zoff + hoff[i], r, false);
-          G[m - R][i] = make_u(r);
+          Raw<T, KIND> r;
+          load_raw<T, KIND>(A, zoff + hoff[i], r, false);
+          G[m - R][i] = stage_input<T, KIND, COMP>(H, r);
         } else {
           G[m - R][i] = mk((T)0, (T)0);
         }
@@ -610,21 +802,21 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
   constexpr int NREAD = NIN + (KI::has_acc ? 1 : 0) + 1;
   constexpr bool kD2Ck4 = KIND == K_CK_4 && P == 1 && !IS_DBL;
   constexpr int D = (NREAD <= GPE_PREFETCH2_MAX || kD2Ck4) ? 2 : 1;
-  Raw rn[D][P];
-  Raw hn[D][HPT];
+  Raw<T, KIND> rn[D][P];
+  Raw<T, KIND> hn[D][HPT];
   cx<T> on[P][NOA];
-  auto issue_raw = [&](int k, Raw *rb, Raw *hb) {
+  auto issue_raw = [&](int k, Raw<T, KIND> *rb, Raw<T, KIND> *hb) {
     const size_t zi = (size_t)bcmap(k + R, nz, per) * plane;
 #pragma unroll
-    for (int p = 0; p < P; ++p) load_raw(zi + roff[p], rb[p], true);
+    for (int p = 0; p < P; ++p) load_raw<T, KIND>(A, zi + roff[p], rb[p], true);
 #pragma unroll
     for (int i = 0; i < HPT; ++i)
-      if (hl[i] >= 0) load_raw(zi + hoff[i], hb[i], false);
+      if (hl[i] >= 0) load_raw<T, KIND>(A, zi + hoff[i], hb[i], false);
   };
   auto issue_out = [&](int k) {
     if constexpr (NO > 0) {
 #pragma unroll
-      for (int p = 0; p < P; ++p) load_out((size_t)k * plane + roff[p], on[p]);
+      for (int p = 0; p < P; ++p) load_out<T, KIND, COMP>(A, (size_t)k * plane + roff[p], on[p]);
     }
   };
 #pragma unroll
@@ -632,21 +824,20 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
     if (z0 + d < z1) issue_raw(z0 + d, rn[d], hn[d]);
   issue_out(z0);
 
-  double acc_norm = 0.0, acc_emax = 0.0, acc_en = 0.0;
-  T thr = (T)-1;  // err_may_lead: every site of the first plane is measured
+  Sums<T> sum;
 
   // one plane of the march; rb/hb hold plane k+R and are refilled with
   // plane k+D+R
-  auto step = [&](const int k, Raw *rb, Raw *hb) {
+  auto step = [&](const int k, Raw<T, KIND> *rb, Raw<T, KIND> *hb) {
     V *Ld = lds[(k - z0) & 1];
     // consume what was prefetched for plane k
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      q[2 * R][p] = make_u(rb[p]);
-      if constexpr (NF > 0) make_F(rb[p], F[R][p]);
+      q[2 * R][p] = stage_input<T, KIND, COMP>(H, rb[p]);
+      if constexpr (NF > 0) out_terms<T, KIND, COMP>(A, rb[p], F[R][p]);
     }
 #pragma unroll
-    for (int i = 0; i < HPT; ++i) G[R][i] = hl[i] >= 0 ? make_u(hb[i]) : mk((T)0, (T)0);
+    for (int i = 0; i < HPT; ++i) G[R][i] = hl[i] >= 0 ? stage_input<T, KIND, COMP>(H, hb[i]) : mk((T)0, (T)0);
     cx<T> oc[P][NOA];
     if constexpr (NO > 0) {
 #pragma unroll
@@ -701,126 +892,8 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
       const bool act = act_x && (gj[p] < ny);
       const size_t s = (size_t)k * plane + (size_t)gj[p] * nx + gi;
 
-      if constexpr (KIND == K_ENERGY) {
-        if (act) {
-          cx<T> pr = cmul(mk(-lap.re, -lap.im), mk(c0.re, -c0.im));
-          T m2;
-          if constexpr (IS_DBL) {
-            m2 = c0.re * c0.re + c0.im * c0.im;
-          } else {
-            const T m = cabs_(c0);
-            m2 = m * m;
-          }
-          acc_en += (double)(pr.re + (T)0.5 * (m2 * m2));
-        }
-      } else {
-        cx<T> dpx = mk((T)0, (T)0);
-        if (A.use_urhs) dpx = d1<T, R>(xm2, xm1, xp1, xp2, div_of(A.d_x), A.inv_x);
-        const cx<T> f = rhs_site<T>(A, c0, lap, dpx, gi, gj[p], k);
-        cx<T> err = mk((T)0, (T)0);
-        bool lead = false;
-        if (act) {
-          if constexpr (KIND == K_RHS || KIND == K_RK2_1 || KIND == K_RK4_1 || KIND == K_RK4_3) {
-            stc<T>(A.kout, s, f);
-          } else if constexpr (KIND == K_RK4_2) {
-            stc<T>(A.kout, s, f);
-            stc<T>(A.acc_out, s, F[0][p][0] + rdiv(f, div_of(A.d3), 1.0 / 3.0));
-          } else if constexpr (KI::is_ck) {
-            cx<T> kk;  // kk = dt*f
-            if constexpr (IS_DBL || !COMP) {
-              kk = cmul(mk((T)A.dtr, (T)A.dti), f);
-            } else {
-              // FP64 dt: no systematic bias from dt rounded to FP32
-              cx<double> kd = cmul(mk(A.dtr, A.dti), todbl(f));
-              kk = mk((T)kd.re, (T)kd.im);
-            }
-            if constexpr (KIND == K_CK_1) {
-              stc<T>(A.kout, s, kk);
-              if constexpr (!COMP) {
-                if (A.write_scale) {
-                  // psi_scal = abs(in) + dt*abs(f) + 1e-30 (solve.f90:176-178)
-                  T af = cabs_(f), au = cabs_(c0);
-                  cx<T> sc = mk((au + (T)A.sdtr * af) + (T)1e-30, (T)A.sdti * af);
-                  if (A.scale_real)
-                    static_cast<T *>(A.scale_out)[s] = sc.re;
-                  else
-                    stc<T>(A.scale_out, s, sc);
-                }
-              }
-            } else if constexpr (KIND < K_CK_6) {
-              stc<T>(A.kout, s, kk);
-            } else {
-              // K_CK_6: new state and the error norm (solve.f90:365-375, 184)
-              err = F[0][p][COMP ? 2 : 1] + rmul((T)ck_dc(6), kk);
-              cx<double> np;
-              if constexpr (IS_DBL) {
-                np = F[0][p][0] + rmul((T)ck_c(6), kk);
-                stc<T>(A.psi_out, s, np);
-              } else if constexpr (COMP) {
-                const cx<double> dl = todbl(F[0][p][1]) + rmul(ck_c(6), todbl(kk));
-                np = (todbl(F[0][p][0]) + todbl(oc[p][0])) + dl;
-                const cx<T> hi = mk((T)np.re, (T)np.im);
-                stc<T>(A.psi_out, s, hi);
-                stc<T>(A.lo_out, s, mk((T)(np.re - (double)hi.re), (T)(np.im - (double)hi.im)));
-              } else {
-                const cx<T> nf = F[0][p][0] + rmul((T)ck_c(6), kk);
-                stc<T>(A.psi_out, s, nf);
-                np = todbl(nf);
-              }
-              // |scale|^2, or in the compensated form its term |psi|^2
-              const cx<T> sc = COMP ? F[0][p][0] : oc[p][0];
-              lead = err_may_lead(err, sc.re * sc.re + sc.im * sc.im, thr);
-              const double wn = wx * wy[p] * nweight(k, nz, A.w1, A.w2, A.w3);
-              acc_norm += wn * (np.re * np.re + np.im * np.im);
-            }
-          } else if constexpr (KI::final_) {
-            // K_EULER, K_RK2_2, K_RK4_4
-            cx<T> ps, incr;  // psi' = ps + dt*incr
-            if constexpr (KIND == K_EULER) {
-              ps = c0;
-              incr = f;
-            } else if constexpr (KIND == K_RK2_2) {
-              ps = F[0][p][0];
-              incr = f;
-            } else {
-              ps = F[0][p][0];
-              incr = F[0][p][1] + rdiv(f, div_of(A.d6), 1.0 / 6.0);
-            }
-            cx<double> np;
-            if constexpr (IS_DBL) {
-              np = ps + cmul(mk((T)A.dtr, (T)A.dti), incr);
-              stc<T>(A.psi_out, s, np);
-            } else if constexpr (COMP) {
-              np = (todbl(ps) + todbl(oc[p][0])) + cmul(mk(A.dtr, A.dti), todbl(incr));
-              const cx<T> hi = mk((T)np.re, (T)np.im);
-              stc<T>(A.psi_out, s, hi);
-              stc<T>(A.lo_out, s, mk((T)(np.re - (double)hi.re), (T)(np.im - (double)hi.im)));
-            } else {
-              const cx<T> nf = ps + cmul(mk((T)A.dtr, (T)A.dti), incr);
-              stc<T>(A.psi_out, s, nf);
-              np = todbl(nf);
-            }
-            const double wn = wx * wy[p] * nweight(k, nz, A.w1, A.w2, A.w3);
-            acc_norm += wn * (np.re * np.re + np.im * np.im);
-          }
-        }
-        if constexpr (KIND == K_CK_6) {
-          if (__any(lead)) {
-            if (lead) {
-              if constexpr (COMP) {
-                // |err/scale|^2, maximised; its square root after the march
-                const double e2 = err_ratio2(err, scale_from_kk1(A, F[0][p][0], F[0][p][NF - 1]));
-                acc_emax = (e2 > acc_emax || e2 != e2) ? e2 : acc_emax;
-              } else {
-                // abs(err/scale) (solve.f90:184), in the storage precision
-                const T e = cabs_(cdiv(err, oc[p][0]));
-                acc_emax = ((double)e > acc_emax || e != e) ? (double)e : acc_emax;
-              }
-            }
-            thr = err_lead<T>(COMP ? sqrt(acc_emax) : acc_emax);
-          }
-        }
-      }
+      emit_site<T, R, KIND, COMP>(A, act, s, gi, gj[p], k, c0, lap, xm2, xm1, xp1, xp2, F[0][p], oc[p],
+                                  wx * wy[p] * nweight(k, nz, A.w1, A.w2, A.w3), sum);
     }
 
     // shift queue and FIFOs
@@ -849,37 +922,7 @@ __device__ __forceinline__ void stage_tile(Args<T> &A, const int tx, const int t
     }
   }
 
-  // The compensated form maximised |err/scale|^2: the maximum of |err/scale|
-  // is its square root (monotone; NaN stays NaN).
-  if constexpr (KIND == K_CK_6 && COMP) acc_emax = sqrt(acc_emax);
-  // Deterministic block reductions: xor-shuffle within the wave, then the
-  // waves in order.
-  if constexpr (KI::final_ || KIND == K_ENERGY) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      acc_norm += __shfl_xor(acc_norm, o);
-      acc_en += __shfl_xor(acc_en, o);
-      double om = __shfl_xor(acc_emax, o);
-      acc_emax = (om > acc_emax || om != om) ? om : acc_emax;
-    }
-    if (lane == 0) {
-      red[0][wave] = acc_norm;
-      red[1][wave] = acc_emax;
-      red[2][wave] = acc_en;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double sn = 0.0, se = 0.0, mx = 0.0;
-      for (int w = 0; w < NW; ++w) {
-        sn += red[0][w];
-        se += red[2][w];
-        mx = (red[1][w] > mx || red[1][w] != red[1][w]) ? red[1][w] : mx;
-      }
-      if (pn) pn[slot] = sn;
-      if (pe) pe[slot] = mx;
-      if (pen) pen[slot] = se;
-    }
-  }
+  block_sums<T, KIND, COMP, NW>(sum, red, slot, pn, pe, pen);
 }
 
 // The kernel's only argument, as a tile of T reads it.
@@ -927,41 +970,6 @@ __global__ void __launch_bounds__(64 * NW)
     if (active[it.inst])
       stage_tile<T, R, NW, P, KIND, COMP>(args_at<T>(insts + it.inst), it.tx, it.ty, it.z0, it.z1, it.slot, pn, pe, nullptr);
     __syncthreads();  // the next item reuses the LDS tile
-  }
-}
-
-// Sum / max of the per-block partials in a fixed order (one workgroup).
-// out[0] = sum(part_norm) * scale_norm, out[1] = max(part_emax) / eps
-// (maxval(...)/eps, solve.f90:184), out[2] = sum(part_energy) * scale_energy;
-// hist (if set) gets out[0].
-static __global__ void __launch_bounds__(256) reduce_partials(const double *pn, const double *pe, const double *pen, int n,
-                                                       double scale_norm, double eps, double scale_energy,
-                                                       double *out, double *hist) {
-  __shared__ double s0[256], s1[256], s2[256];
-  double a = 0.0, m = 0.0, c = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) {
-    if (pn) a += pn[i];
-    if (pe) m = (pe[i] > m || pe[i] != pe[i]) ? pe[i] : m;
-    if (pen) c += pen[i];
-  }
-  s0[threadIdx.x] = a;
-  s1[threadIdx.x] = m;
-  s2[threadIdx.x] = c;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      s0[threadIdx.x] += s0[threadIdx.x + w];
-      double o = s1[threadIdx.x + w];
-      s1[threadIdx.x] = (o > s1[threadIdx.x] || o != o) ? o : s1[threadIdx.x];
-      s2[threadIdx.x] += s2[threadIdx.x + w];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    out[0] = s0[0] * scale_norm;
-    out[1] = s1[0] / eps;
-    out[2] = s2[0] * scale_energy;
-    if (hist) *hist = out[0];
   }
 }
 
