@@ -551,6 +551,7 @@ int gpe_batch_create(int64_t hbm_budget, gpe_batch **out) {
     delete b;
     return fail(GPE_EHIP, "hipStreamCreate failed");
   }
+  transfers_retain();
   bool ok = hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) == hipSuccess;
   for (int q = 0; q < kAuxStreams && ok; ++q) ok = hipStreamCreateWithFlags(&b->aux[q], hipStreamNonBlocking) == hipSuccess;
   for (int q = 0; q < kMaxGroups && ok; ++q) ok = hipEventCreateWithFlags(&b->ev_done[q], hipEventDisableTiming) == hipSuccess;
@@ -592,6 +593,7 @@ void gpe_batch_destroy(gpe_batch *b) {
   if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
+  transfers_release();
 }
 
 int gpe_batch_footprint(const gpe_params *params, int64_t *bytes) {

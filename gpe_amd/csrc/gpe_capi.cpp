@@ -670,6 +670,7 @@ int gpe_ctx_create(const gpe_params *params, gpe_ctx **out) {
     c->hscal[3] = 0.0;
   }
   fill_base(params, c->prec, c->base);
+  transfers_retain();
   *out = c;
   return GPE_OK;
 bad:
@@ -683,6 +684,7 @@ void gpe_ctx_destroy(gpe_ctx *ctx) {
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   free_all(ctx);
   delete ctx;
+  transfers_release();
 }
 
 int gpe_sim_upload(gpe_ctx *c, const void *psi, int32_t host_type) {
@@ -1017,16 +1019,7 @@ int gpe_sim_filtered(gpe_ctx *c, double filter_kc, double m, void *out, int32_t 
   double2 *a = static_cast<double2 *>(c->spec);
   if (int rc = spectral_filter(c->P.nx, c->P.ny, c->P.nz, a, m, filter_kc, c->stream)) return rc;
   HIPCHK(hipStreamSynchronize(c->stream));
-  if (host_type == GPE_HOST_C128) {
-    if (int rc = field_download(GPE_FP64, (size_t)c->P.nx * c->P.ny, c->P.nz, a, nullptr, out, host_type)) return rc;
-  } else {
-    // the filtered field is FP64: round it to complex64 on the host
-    std::vector<double> tmp(2 * c->n);
-    if (int rc = field_download(GPE_FP64, (size_t)c->P.nx * c->P.ny, c->P.nz, a, nullptr, tmp.data(), GPE_HOST_C128))
-      return rc;
-    float *o = static_cast<float *>(out);
-    for (size_t q = 0; q < 2 * c->n; ++q) o[q] = (float)tmp[q];
-  }
+  if (int rc = words_download(16, c->n, a, nullptr, out, host_type)) return rc;
   if (length) return linelength_of(c, GPE_FP64, a, nullptr, length);
   return GPE_OK;
 }
@@ -1146,20 +1139,9 @@ int gpe_sim_rhs(gpe_ctx *c, void *out, int32_t host_type) {
   int rc = run_kind(c, K_RHS, A);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(c->stream));
-  if (c->prec == GPE_FP64) {
-    if (host_type != GPE_HOST_C128) return fail(GPE_EINVAL, "FP64 context returns complex128 host data");
-    HIPCHK(hipMemcpy(out, tmp, c->n * 16, hipMemcpyDeviceToHost));
-  } else {
-    if (host_type == GPE_HOST_C64) {
-      HIPCHK(hipMemcpy(out, tmp, c->n * 8, hipMemcpyDeviceToHost));
-    } else {
-      std::vector<float> f(2 * c->n);
-      HIPCHK(hipMemcpy(f.data(), tmp, c->n * 8, hipMemcpyDeviceToHost));
-      double *d = (double *)out;
-      for (size_t q = 0; q < 2 * c->n; ++q) d[q] = f[q];
-    }
-  }
-  return GPE_OK;
+  if (c->prec == GPE_FP64 && host_type != GPE_HOST_C128)
+    return fail(GPE_EINVAL, "FP64 context returns complex128 host data");
+  return words_download((int)c->esz, c->n, tmp, nullptr, out, host_type == GPE_HOST_C64 ? host_type : GPE_HOST_C128);
 }
 
 int gpe_solver_step(gpe_ctx *c, const void *var_in, int32_t halo, void *var_out, gpe_step_state *st) {

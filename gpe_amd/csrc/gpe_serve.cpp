@@ -18,6 +18,7 @@
 #include <cstring>
 #include <deque>
 #include <map>
+#include <memory>
 #include <new>
 #include <string>
 #include <utility>
@@ -30,12 +31,34 @@ using gpe::fail;
 
 namespace {
 
+// A host field, its memory not written before the field is.
+struct HostBytes {
+  std::unique_ptr<unsigned char[]> p;
+  size_t n = 0;
+  bool alloc(size_t bytes) {
+    p.reset(new (std::nothrow) unsigned char[bytes]);
+    n = p ? bytes : 0;
+    return p != nullptr;
+  }
+  void clear() {
+    p.reset();
+    n = 0;
+  }
+  bool empty() const { return n == 0; }
+};
+
+void host_copy(void *dst, const void *src, size_t bytes) {
+  gpe::host_parts(bytes, [&](size_t a, size_t b) {
+    std::memcpy(static_cast<char *>(dst) + a, static_cast<const char *>(src) + a, b - a);
+  });
+}
+
 struct Request {
   int64_t ticket = 0;
   gpe_params P{};
   gpe_step_state st{};
   int64_t nsteps = 0;
-  std::vector<unsigned char> field;  // host copy of the initial field (empty: random phase)
+  HostBytes field;  // host copy of the initial field (empty: random phase)
   int32_t host_type = GPE_HOST_C128;
   uint64_t seed = 0;
   double kmax = 0.0;
@@ -46,7 +69,7 @@ struct Result {
   int32_t status = 0;
   gpe_step_state st{};
   gpe_params P{};
-  std::vector<unsigned char> field;  // complex128
+  HostBytes field;  // complex128
 };
 
 size_t sites_of(const gpe_params &P) { return (size_t)P.nx * (size_t)P.ny * (size_t)P.nz; }
@@ -114,11 +137,8 @@ int gpe_serve_submit(gpe_serve *s, const gpe_params *params, const void *psi, in
   if (psi) {
     if (host_type != GPE_HOST_C128 && host_type != GPE_HOST_C64) return fail(GPE_EINVAL, "host_type");
     const size_t nb = (size_t)r.sites * (host_type == GPE_HOST_C128 ? 16 : 8);
-    try {
-      r.field.assign(static_cast<const unsigned char *>(psi), static_cast<const unsigned char *>(psi) + nb);
-    } catch (const std::bad_alloc &) {
-      return fail(GPE_ENOMEM, "host copy of the initial field (%zu bytes)", nb);
-    }
+    if (!r.field.alloc(nb)) return fail(GPE_ENOMEM, "host copy of the initial field (%zu bytes)", nb);
+    host_copy(r.field.p.get(), psi, nb);
     r.host_type = host_type;
   } else {
     if (!(kmax > 0.0)) return fail(GPE_EINVAL, "random-phase request needs kmax > 0");
@@ -144,7 +164,7 @@ int gpe_serve_step(gpe_serve *s, int32_t iterations, int32_t *running, int32_t *
     if (r.field.empty())
       rc = gpe_batch_add_random_phase(s->batch, &r.P, r.seed, r.kmax, &r.st, r.nsteps, &id);
     else
-      rc = gpe_batch_add(s->batch, &r.P, r.field.data(), r.host_type, &r.st, r.nsteps, &id);
+      rc = gpe_batch_add(s->batch, &r.P, r.field.p.get(), r.host_type, &r.st, r.nsteps, &id);
     if (rc == GPE_EFULL) break;  // waits for memory
     if (rc) {
       // cannot be admitted at all (e.g. a device error building its state):
@@ -162,7 +182,6 @@ int gpe_serve_step(gpe_serve *s, int32_t iterations, int32_t *running, int32_t *
     }
     s->resident_sites += r.sites;
     r.field.clear();
-    r.field.shrink_to_fit();
     s->running.emplace(id, std::move(r));
     s->queue.pop_front();
   }
@@ -186,13 +205,9 @@ int gpe_serve_step(gpe_serve *s, int32_t iterations, int32_t *running, int32_t *
     res.P = it->second.P;
     res.st = it->second.st;
     rc = GPE_OK;
-    try {
-      res.field.resize(sites_of(res.P) * 16);
-    } catch (const std::bad_alloc &) {
-      rc = fail(GPE_ENOMEM, "host copy of a result");
-    }
+    if (!res.field.alloc(sites_of(res.P) * 16)) rc = fail(GPE_ENOMEM, "host copy of a result");
     if (!rc) rc = gpe_batch_query(s->batch, ids[i], &res.st, nullptr, nullptr, nullptr, nullptr);
-    if (!rc) rc = gpe_batch_download(s->batch, ids[i], res.field.data(), GPE_HOST_C128);
+    if (!rc) rc = gpe_batch_download(s->batch, ids[i], res.field.p.get(), GPE_HOST_C128);
     const int rc_remove = gpe_batch_remove(s->batch, ids[i]);
     if (!rc) rc = rc_remove;
     if (rc) {
@@ -240,12 +255,14 @@ int gpe_serve_result(gpe_serve *s, int64_t ticket, void *psi, int32_t host_type,
     return fail(GPE_ESTATE, "request %lld has no field (status %d)", (long long)ticket, status);
   }
   const size_t n = sites_of(r.P);
-  const double *src = reinterpret_cast<const double *>(r.field.data());
+  const double *src = reinterpret_cast<const double *>(r.field.p.get());
   if (host_type == GPE_HOST_C128) {
-    std::memcpy(psi, src, n * 16);
+    host_copy(psi, src, n * 16);
   } else if (host_type == GPE_HOST_C64) {
     float *d = static_cast<float *>(psi);
-    for (size_t i = 0; i < 2 * n; ++i) d[i] = (float)src[i];
+    gpe::host_parts(n * 16, [&](size_t a, size_t b) {
+      for (size_t i = a / 8; i < b / 8; ++i) d[i] = (float)src[i];
+    });
   } else {
     return fail(GPE_EINVAL, "host_type");
   }

@@ -1,7 +1,6 @@
 // host_common.cpp -- host helpers shared by the single-simulation and the
-// batch entry points: the launch descriptor's constant part and field
-// conversions between host arrays and device storage (error reporting is
-// in errors.cpp).
+// batch entry points: the launch descriptor's constant part (field transfers
+// are in transfer.hip, error reporting in errors.cpp).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -71,85 +70,5 @@ void fill_base(const gpe_params *params, int prec, StageArgs &A) {
   A.w2 = 7.0 / 6.0;
   A.w3 = 23.0 / 24.0;
   }
-
-}  // namespace gpe
-
-namespace gpe {
-
-// Host array -> device storage.  src_pitch_planes: elements between
-// z-planes of the host array; row_off: element offset of the interior's
-// (0, 0, 0).  FP32 forms from complex128 split each value into hi = fl32(v)
-// and lo = fl32(v - hi); complex64 into a compensated form sets lo = 0.
-int field_upload(int prec, size_t plane, int nz, const void *src, int host_type, size_t src_pitch_planes,
-                 size_t row_off, void *hi, void *lo) {
-  const size_t n = plane * (size_t)nz;
-  const bool contiguous = src_pitch_planes == plane && row_off == 0;
-  const bool comp = prec == GPE_FP32C;
-  if (host_type != GPE_HOST_C128 && host_type != GPE_HOST_C64) return fail(GPE_EINVAL, "unsupported host type");
-  if (prec == GPE_FP64) {
-    if (host_type != GPE_HOST_C128) return fail(GPE_EINVAL, "FP64 storage takes complex128 host data");
-    if (contiguous) {
-      GPE_HIPCHK(hipMemcpy(hi, src, n * 16, hipMemcpyHostToDevice));
-    } else {
-      GPE_HIPCHK(hipMemcpy2D(hi, plane * 16, (const char *)src + row_off * 16, src_pitch_planes * 16, plane * 16,
-                             nz, hipMemcpyHostToDevice));
-    }
-    return GPE_OK;
-  }
-  if (host_type == GPE_HOST_C64) {
-    if (contiguous) {
-      GPE_HIPCHK(hipMemcpy(hi, src, n * 8, hipMemcpyHostToDevice));
-    } else {
-      GPE_HIPCHK(hipMemcpy2D(hi, plane * 8, (const char *)src + row_off * 8, src_pitch_planes * 8, plane * 8, nz,
-                             hipMemcpyHostToDevice));
-    }
-    if (comp) GPE_HIPCHK(hipMemset(lo, 0, n * 8));
-    return GPE_OK;
-  }
-  std::vector<float> h(2 * plane), l(2 * plane);
-  for (int k = 0; k < nz; ++k) {
-    const double *s = (const double *)src + 2 * (row_off + (size_t)k * src_pitch_planes);
-    for (size_t q = 0; q < 2 * plane; ++q) {
-      const float v = (float)s[q];
-      h[q] = v;
-      l[q] = (float)(s[q] - (double)v);
-    }
-    GPE_HIPCHK(hipMemcpy((char *)hi + (size_t)k * plane * 8, h.data(), plane * 8, hipMemcpyHostToDevice));
-    if (comp) GPE_HIPCHK(hipMemcpy((char *)lo + (size_t)k * plane * 8, l.data(), plane * 8, hipMemcpyHostToDevice));
-  }
-  return GPE_OK;
-}
-
-// Device storage -> contiguous host array (complex128 gets hi + lo in
-// double; complex64 gets fl32(hi + lo)).  The caller orders this after the
-// kernels that wrote the field.
-int field_download(int prec, size_t plane, int nz, const void *hi, const void *lo, void *dst, int host_type) {
-  const size_t n = plane * (size_t)nz;
-  const bool comp = prec == GPE_FP32C;
-  if (host_type != GPE_HOST_C128 && host_type != GPE_HOST_C64) return fail(GPE_EINVAL, "unsupported host type");
-  if (prec == GPE_FP64) {
-    if (host_type != GPE_HOST_C128) return fail(GPE_EINVAL, "FP64 storage returns complex128 host data");
-    GPE_HIPCHK(hipMemcpy(dst, hi, n * 16, hipMemcpyDeviceToHost));
-    return GPE_OK;
-  }
-  if (host_type == GPE_HOST_C64 && !comp) {
-    GPE_HIPCHK(hipMemcpy(dst, hi, n * 8, hipMemcpyDeviceToHost));
-    return GPE_OK;
-  }
-  std::vector<float> h(2 * plane), l(2 * plane, 0.f);
-  for (int k = 0; k < nz; ++k) {
-    GPE_HIPCHK(hipMemcpy(h.data(), (const char *)hi + (size_t)k * plane * 8, plane * 8, hipMemcpyDeviceToHost));
-    if (comp)
-      GPE_HIPCHK(hipMemcpy(l.data(), (const char *)lo + (size_t)k * plane * 8, plane * 8, hipMemcpyDeviceToHost));
-    if (host_type == GPE_HOST_C128) {
-      double *d = (double *)dst + 2 * (size_t)k * plane;
-      for (size_t q = 0; q < 2 * plane; ++q) d[q] = (double)h[q] + (double)l[q];
-    } else {
-      float *d = (float *)dst + 2 * (size_t)k * plane;
-      for (size_t q = 0; q < 2 * plane; ++q) d[q] = (float)((double)h[q] + (double)l[q]);
-    }
-  }
-  return GPE_OK;
-}
 
 }  // namespace gpe

@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -27,6 +28,15 @@ void fill_base(const gpe_params *params, int prec, StageArgs &A);
 int field_upload(int prec, size_t plane, int nz, const void *src, int host_type, size_t src_pitch_planes,
                  size_t row_off, void *hi, void *lo);
 int field_download(int prec, size_t plane, int nz, const void *hi, const void *lo, void *dst, int host_type);
+// `sites` complex values of `stored` bytes (16 or 8; lo: the low words of the
+// compensated form, or null) into a host array.
+int words_download(int stored, size_t sites, const void *hi, const void *lo, void *dst, int host_type);
+// f(begin, end) over the bytes of a host array, by several threads where its
+// size is worth them.
+void host_parts(size_t bytes, const std::function<void(size_t, size_t)> &f);
+// The staging buffers of these transfers are kept while somebody retains them.
+void transfers_retain();
+void transfers_release();
 extern thread_local std::string g_err;
 
 // A roctx range for the lifetime of the object (rocprofv3 --marker-trace
