@@ -37,6 +37,7 @@ UNITS = [("gpe_misc.hip", "gpe_misc", ["-ffp-contract=off"]),
          ("gpe_batch.cpp", "gpe_batch", ["-ffp-contract=off", "-x", "hip"]),
          ("host_common.cpp", "host_common", ["-ffp-contract=off", "-x", "hip"]),
          ("transfer.hip", "transfer", ["-ffp-contract=off"]),
+         ("gpe_diag.hip", "gpe_diag", ["-ffp-contract=off"]),
          ("gpe_ic.cpp", "gpe_ic", ["-ffp-contract=off", "-x", "hip"]),
          ("tune_table.cpp", "tune_table", ["-x", "hip"]),
          ("gpe_spectral.cpp", "gpe_spectral", ["-ffp-contract=off", "-x", "hip"]),

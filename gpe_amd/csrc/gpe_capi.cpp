@@ -21,6 +21,7 @@
 
 #include "../../include/gpe_hip.h"
 #include "host_common.h"
+#include "gpe_diag.h"
 #include "gpe_ic.h"
 #include "gpe_spectral.h"
 #include "launch.h"
@@ -138,11 +139,7 @@ struct gpe_ctx {
   std::vector<Ev> pending;
   std::vector<hipEvent_t> pool;
   int64_t prof_n[GPE_PROF_KINDS] = {};
-  // line-length point lists (grown on demand)
-  void *ll_buf = nullptr;
-  int ll_cap = 0;
-  void *zr_buf = nullptr;  // zeros pass: cap points + a counter
-  int zr_cap = 0;
+  DiagWork diag;  // lists of the vortex diagnostics
   // FFT-side diagnostics: a complex128 field and small scratch (on demand)
   void *spec = nullptr, *spec_aux = nullptr;
   double prof_ms[GPE_PROF_KINDS] = {};
@@ -539,7 +536,7 @@ int solver_call(gpe_ctx *c, double *hist_slot) {
 
 void free_all(gpe_ctx *c) {
   void *ptrs[] = {c->psi, c->psi2, c->lo, c->lo2, c->k[0], c->k[1], c->k[2], c->k[3], c->k[4], c->k[5],
-                  c->acc, c->scale, c->part, c->hpart, c->hist, c->ll_buf, c->zr_buf, c->spec, c->spec_aux};
+                  c->acc, c->scale, c->part, c->hpart, c->hist, c->spec, c->spec_aux};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (c->hscal) (void)hipHostFree(c->hscal);
@@ -790,42 +787,6 @@ int gpe_sim_energy(gpe_ctx *c, double *energy) {
 
 }  // extern "C"
 
-namespace {
-// Segment of a one-point cell to the latest earlier second point, with the
-// reference's face/edge weights (variables.f90:1140-1153), in T.
-template <typename T>
-T ll_segment_host(T x1, T y1, T z1, T x2, T y2, T z2) {
-  auto in01 = [](T v) { return v == (T)0 || v == (T)1; };
-  T a = (T)1;
-  const bool ex = x1 == x2 && in01(x1), ey = y1 == y2 && in01(y1), ez = z1 == z2 && in01(z1);
-  if (ex || ey) {
-    a = a * (T)0.5;
-    if ((ex && ey) || (ey && ez)) a = a * (T)0.5;
-  }
-  return a * std::sqrt((x1 - x2) * (x1 - x2) + (y1 - y2) * (y1 - y2) + (z1 - z2) * (z1 - z2));
-}
-
-template <typename T>
-double ll_singles(std::vector<LinePoint> &w, std::vector<LinePoint> &s) {
-  auto by_cell = [](const LinePoint &a, const LinePoint &b) { return a.cell < b.cell; };
-  std::sort(w.begin(), w.end(), by_cell);
-  std::sort(s.begin(), s.end(), by_cell);
-  double sum = 0.0;
-  T x2 = 0, y2 = 0, z2 = 0;  // before any cell stored a second point
-  size_t j = 0;
-  for (const LinePoint &p : s) {
-    while (j < w.size() && w[j].cell < p.cell) {
-      x2 = (T)w[j].x;
-      y2 = (T)w[j].y;
-      z2 = (T)w[j].z;
-      ++j;
-    }
-    sum += (double)ll_segment_host<T>((T)p.x, (T)p.y, (T)p.z, x2, y2, z2);
-  }
-  return sum;
-}
-}  // namespace
-
 extern "C" {
 
 int gpe_sim_hamiltonian(gpe_ctx *c, double *h) {
@@ -835,20 +796,20 @@ int gpe_sim_hamiltonian(gpe_ctx *c, double *h) {
   if (c->part_cap < PW_BLOCKS) return fail(GPE_EINVAL, "internal: partial buffer below %d", PW_BLOCKS);
   double E = 0.0;
   if (int rc = gpe_sim_energy(c, &E)) return rc;
-  double *p2 = c->part, *p4 = c->part + c->part_cap, *pv = c->part + 2 * (size_t)c->part_cap;
+  double *p2 = c->part, *p4 = c->part + PW_BLOCKS, *pv = c->part + 2 * PW_BLOCKS;  // part holds 3 part_cap
   // sums of |psi|^2, |psi|^4 and V |psi|^2 over the field (hi + lo in the
   // compensated form)
   auto moments = [&](const void *lo, double &s2, double &s4, double &sv) -> int {
     hipError_t e = launch_moments(c->prec == GPE_FP64 ? 0 : 1, c->psi, lo, c->base, p2, p4, pv, c->stream);
     if (e != hipSuccess) return fail(GPE_EHIP, "moments launch: %s", hipGetErrorString(e));
-    std::vector<double> hp(3 * (size_t)c->part_cap);
-    HIPCHK(hipMemcpyAsync(hp.data(), c->part, sizeof(double) * hp.size(), hipMemcpyDeviceToHost, c->stream));
+    double hp[3 * PW_BLOCKS];
+    HIPCHK(hipMemcpyAsync(hp, c->part, sizeof hp, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     s2 = s4 = sv = 0.0;
     for (int b = 0; b < PW_BLOCKS; ++b) {
       s2 += hp[b];
-      s4 += hp[c->part_cap + b];
-      sv += hp[2 * (size_t)c->part_cap + b];
+      s4 += hp[PW_BLOCKS + b];
+      sv += hp[2 * PW_BLOCKS + b];
     }
     return GPE_OK;
   };
@@ -869,77 +830,32 @@ int gpe_sim_hamiltonian(gpe_ctx *c, double *h) {
   return GPE_OK;
 }
 
-}  // extern "C"
-
-namespace {
-int linelength_of(gpe_ctx *c, int prec, const void *psi, const void *lo, double *length);
-}  // namespace
-
-extern "C" {
-
 int gpe_sim_linelength(gpe_ctx *c, double *length) {
   if (!c || !length) return fail(GPE_EINVAL, "NULL argument");
   if (!c->uploaded) return fail(GPE_ESTATE, "no field uploaded");
-  return linelength_of(c, c->prec, c->psi, c->comp ? c->lo : nullptr, length);
+  return diag_linelength(c->diag, c->prec, c->psi, c->comp ? c->lo : nullptr, c->P.nx, c->P.ny, c->P.nz, c->P.dx, length,
+                         c->stream);
 }
 
 }  // extern "C"
 
 namespace {
-// linelength (variables.f90:896-1162) of a device field of the context's
-// grid in storage form prec (lo: the compensated low word or NULL).
-int linelength_of(gpe_ctx *c, int prec, const void *psi, const void *lo, double *length) {
-  const long long ncell = (long long)(c->P.nx - 2) * (c->P.ny - 2) * (c->P.nz - 2);
-  const int nb = (int)std::min<long long>((ncell + 255) / 256, std::min(c->part_cap, 2048));
-  int cnt[2] = {0, 0};
-  for (;;) {
-    if (!c->ll_buf || c->ll_cap < 1) {
-      const int cap = c->ll_cap > 0 ? c->ll_cap : (1 << 16);
-      if (c->ll_buf) (void)hipFree(c->ll_buf);
-      c->ll_buf = nullptr;
-      if (hipMalloc(&c->ll_buf, 2 * sizeof(LinePoint) * (size_t)cap + 256) != hipSuccess)
-        return fail(GPE_ENOMEM, "line-length lists of %d points", cap);
-      c->ll_cap = cap;
-    }
-    LinePoint *w = (LinePoint *)c->ll_buf, *sg = w + c->ll_cap;
-    int *counts = (int *)(sg + c->ll_cap);
-    HIPCHK(hipMemsetAsync(counts, 0, 2 * sizeof(int), c->stream));
-    hipError_t e = launch_linelength(prec, psi, lo, c->P.nx, c->P.ny, c->P.nz, c->part, nb, w, sg, counts, c->ll_cap,
-                                     c->stream);
-    if (e != hipSuccess) return fail(GPE_EHIP, "linelength launch: %s", hipGetErrorString(e));
-    HIPCHK(hipMemcpyAsync(cnt, counts, sizeof cnt, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const int need = std::max(cnt[0], cnt[1]);
-    if (need <= c->ll_cap) break;
-    // lists overflowed: grow them and run the pass again
-    (void)hipFree(c->ll_buf);
-    c->ll_buf = nullptr;
-    c->ll_cap = need + need / 4;
-  }
-  std::vector<double> part(nb);
-  std::vector<LinePoint> w(cnt[0]), sg(cnt[1]);
-  LinePoint *dw = (LinePoint *)c->ll_buf;
-  HIPCHK(hipMemcpy(part.data(), c->part, sizeof(double) * nb, hipMemcpyDeviceToHost));
-  if (cnt[0]) HIPCHK(hipMemcpy(w.data(), dw, sizeof(LinePoint) * cnt[0], hipMemcpyDeviceToHost));
-  if (cnt[1]) HIPCHK(hipMemcpy(sg.data(), dw + c->ll_cap, sizeof(LinePoint) * cnt[1], hipMemcpyDeviceToHost));
-  double sum = 0.0;
-  for (double v : part) sum += v;
-  sum += prec == GPE_FP32 ? ll_singles<float>(w, sg) : ll_singles<double>(w, sg);
-  *length = prec == GPE_FP32 ? (double)((float)sum * (float)c->P.dx) : sum * c->P.dx;
-  return GPE_OK;
-}
-
-// The unitary forward DFT of the resident field into c->spec.
-int spectral_of_field(gpe_ctx *c) {
-  if (!c->spec && hipMalloc(&c->spec, c->n * 16) != hipSuccess) {
-    c->spec = nullptr;
-    return fail(GPE_ENOMEM, "spectral work field of %zu bytes", c->n * 16);
-  }
+int spectral_scratch(gpe_ctx *c) {
   if (!c->spec_aux &&
       hipMalloc(&c->spec_aux, sizeof(double) * spectral_scratch_doubles(c->P.nx, c->P.ny, c->P.nz)) != hipSuccess) {
     c->spec_aux = nullptr;
     return fail(GPE_ENOMEM, "spectral scratch");
   }
+  return GPE_OK;
+}
+
+// The unscaled forward DFT of the resident field into c->spec.
+int spectral_of_field(gpe_ctx *c) {
+  if (!c->spec && hipMalloc(&c->spec, c->n * 16) != hipSuccess) {
+    c->spec = nullptr;
+    return fail(GPE_ENOMEM, "spectral work field of %zu bytes", c->n * 16);
+  }
+  if (int rc = spectral_scratch(c)) return rc;
   return spectral_forward(c->P.nx, c->P.ny, c->P.nz, c->prec, c->psi, c->comp ? c->lo : nullptr,
                           static_cast<double2 *>(c->spec), c->stream);
 }
@@ -954,11 +870,12 @@ int gpe_sim_condensed_particles(gpe_ctx *c, gpe_condensed *out) {
   if (c->P.nx < 2) return fail(GPE_EINVAL, "condensed_particles needs nx >= 2");
   double M = 0.0;
   if (int rc = gpe_sim_mass(c, &M)) return rc;
-  if (int rc = spectral_of_field(c)) return rc;
-  double2 a0;
-  HIPCHK(hipMemcpyAsync(&a0, c->spec, sizeof a0, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  const double m0 = std::hypot(a0.x, a0.y);
+  if (int rc = spectral_scratch(c)) return rc;
+  double re = 0.0, im = 0.0;
+  if (int rc = spectral_zero_mode(c->n, c->prec, c->psi, c->comp ? c->lo : nullptr, static_cast<double *>(c->spec_aux),
+                                  &re, &im, c->stream))
+    return rc;
+  const double m0 = std::hypot(re, im);
   const double n0 = m0 * m0;
   const double V = (double)c->n;
   const double rho0 = n0 / V;
@@ -1020,7 +937,7 @@ int gpe_sim_filtered(gpe_ctx *c, double filter_kc, double m, void *out, int32_t 
   if (int rc = spectral_filter(c->P.nx, c->P.ny, c->P.nz, a, m, filter_kc, c->stream)) return rc;
   HIPCHK(hipStreamSynchronize(c->stream));
   if (int rc = words_download(16, c->n, a, nullptr, out, host_type)) return rc;
-  if (length) return linelength_of(c, GPE_FP64, a, nullptr, length);
+  if (length) return diag_linelength(c->diag, GPE_FP64, a, nullptr, c->P.nx, c->P.ny, c->P.nz, c->P.dx, length, c->stream);
   return GPE_OK;
 }
 
@@ -1078,41 +995,12 @@ int gpe_sim_zeros(gpe_ctx *c, int32_t which, gpe_zero_point *out, int64_t cap, i
   if (cap < 0 || (cap > 0 && !out)) return fail(GPE_EINVAL, "bad output buffer");
   if (!c->uploaded) return fail(GPE_ESTATE, "no field uploaded");
   static_assert(sizeof(gpe_zero_point) == sizeof(ZeroPoint), "gpe_zero_point layout");
-  const long long ncell = (long long)(c->P.nx - 2) * (c->P.ny - 2) * (c->P.nz - 2);
-  const int nb = (int)std::max<long long>(1, std::min<long long>((ncell + 255) / 256, 4096));
   const double xyzl[3] = {c->P.xl, c->P.yl, c->P.zl}, dxyz[3] = {c->P.dx, c->P.dy, c->P.dz};
-  int cnt = 0;
-  for (;;) {
-    if (!c->zr_buf) {
-      const int zc = c->zr_cap > 0 ? c->zr_cap : (1 << 16);
-      if (hipMalloc(&c->zr_buf, sizeof(ZeroPoint) * (size_t)zc + 256) != hipSuccess)
-        return fail(GPE_ENOMEM, "zero list of %d points", zc);
-      c->zr_cap = zc;
-    }
-    ZeroPoint *pts = (ZeroPoint *)c->zr_buf;
-    int *counter = (int *)(pts + c->zr_cap);
-    HIPCHK(hipMemsetAsync(counter, 0, sizeof(int), c->stream));
-    hipError_t e = launch_zeros(c->prec, c->psi, c->comp ? c->lo : nullptr, c->P.nx, c->P.ny, c->P.nz, xyzl, dxyz,
-                                which, pts, counter, c->zr_cap, nb, c->stream);
-    if (e != hipSuccess) return fail(GPE_EHIP, "zeros launch: %s", hipGetErrorString(e));
-    HIPCHK(hipMemcpyAsync(&cnt, counter, sizeof cnt, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (cnt <= c->zr_cap) break;
-    // the list overflowed: grow it and run the pass again
-    if (cnt > (1 << 28)) return fail(GPE_ENOMEM, "%d zero points", cnt);
-    (void)hipFree(c->zr_buf);
-    c->zr_buf = nullptr;
-    c->zr_cap = cnt + cnt / 4;
-  }
-  std::vector<ZeroPoint> h(cnt);
-  if (cnt) HIPCHK(hipMemcpy(h.data(), c->zr_buf, sizeof(ZeroPoint) * (size_t)cnt, hipMemcpyDeviceToHost));
-  // the reference's file order: section, then k, j, i
-  std::sort(h.begin(), h.end(), [](const ZeroPoint &a, const ZeroPoint &b) {
-    return a.section != b.section ? a.section < b.section : a.cell < b.cell;
-  });
-  const int64_t nout = std::min<int64_t>(cap, cnt);
-  if (nout) std::memcpy(out, h.data(), sizeof(ZeroPoint) * (size_t)nout);
-  *count = cnt;
+  long long found = 0;
+  if (int rc = diag_zeros(c->diag, c->prec, c->psi, c->comp ? c->lo : nullptr, c->P.nx, c->P.ny, c->P.nz, xyzl, dxyz,
+                          which, reinterpret_cast<ZeroPoint *>(out), cap, &found, c->stream))
+    return rc;
+  *count = found;
   return GPE_OK;
 }
 

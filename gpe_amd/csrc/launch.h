@@ -180,18 +180,6 @@ hipError_t launch_norm_f32(const void *psi, const void *lo, int nx, int ny, int 
 hipError_t launch_renorm_f64(void *psi, size_t n, double a, DivC b, hipStream_t s);
 hipError_t launch_renorm_f32(void *psi, void *lo, size_t n, double a, double b, hipStream_t s);
 
-// Vortex-line length cells (diag.hpp): prec GPE_FP64 / GPE_FP32 / GPE_FP32C
-// (lo = low word for the compensated form); nblocks partial sums into part.
-hipError_t launch_linelength(int prec, const void *psi, const void *lo, int nx, int ny, int nz, double *part,
-                             int nblocks, LinePoint *writers, LinePoint *singles, int *counts, int cap,
-                             hipStream_t s);
-
-// Vortex-core points (diag.hpp): which = 0 zeros, 1 re_zeros, 2 im_zeros;
-// appends up to cap points to out and counts all of them in *count.
-hipError_t launch_zeros(int prec, const void *psi, const void *lo, int nx, int ny, int nz, const double *xyzl,
-                        const double *dxyz, int which, ZeroPoint *out, int *count, int cap, int nblocks,
-                        hipStream_t s);
-
 // imprint_vortex_line over the whole field (pointwise.hpp); prec as
 // GPE_FP64 / GPE_FP32 / GPE_FP32C (lo = low word of the compensated form).
 hipError_t launch_imprint(int prec, void *psi, void *lo, const LineArgs &L, hipStream_t s);

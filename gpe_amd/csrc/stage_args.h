@@ -133,12 +133,6 @@ struct InstCtl {
   void *buf[2], *lob[2];
 };
 
-// A zero point of the vortex-line length pass (see diag.hpp).
-struct LinePoint {
-  long long cell;  // linear cell index, x fastest
-  double x, y, z;
-};
-
 // A vortex line to imprint (type line_param, parameters.in:33-43) on a
 // grid, with the reference's safe wavelengths already applied.
 struct LineArgs {

@@ -196,14 +196,15 @@ class Simulation:
         (section, cell, x, y, z) in file order."""
         w = _lib.ZERO_FILES[which]
         n = ctypes.c_int64()
-        _lib.check(self._L.gpe_sim_zeros(self._ctx, w, None, 0, ctypes.byref(n)))
-        out = np.zeros(max(n.value, 1), dtype=_lib.ZERO_DTYPE)
-        m = ctypes.c_int64()
-        _lib.check(self._L.gpe_sim_zeros(self._ctx, w, out.ctypes.data_as(ctypes.c_void_p), n.value,
-                                         ctypes.byref(m)))
-        if m.value != n.value:
-            raise RuntimeError("zero count changed between calls: %d, %d" % (n.value, m.value))
-        return out[:n.value]
+        # room for a dense tangle's points (memory that is not written costs
+        # nothing); more than that are counted first and fetched again
+        cap = max(1024, self.cfg.nx * self.cfg.ny * self.cfg.nz // 16)
+        while True:
+            out = np.empty(cap, dtype=_lib.ZERO_DTYPE)
+            _lib.check(self._L.gpe_sim_zeros(self._ctx, w, out.ctypes.data_as(ctypes.c_void_p), cap, ctypes.byref(n)))
+            if n.value <= cap:
+                return out[:n.value]
+            cap = n.value
 
     def save_zeros(self, proc_dir):
         """zeros<p>.dat, re_zeros<p>.dat and im_zeros<p>.dat of the resident
