@@ -79,18 +79,9 @@ class Team {
     cv_.notify_all();
     for (std::thread &t : th_) t.join();
   }
-  void start() {
-    cpu_set_t set;
-    int cpus = kThreads;
-    if (sched_getaffinity(0, sizeof set, &set) == 0) cpus = CPU_COUNT(&set);
-    try {
-      for (int i = 1; i < std::min(kThreads, cpus); ++i) th_.emplace_back([this, i] { work(i); });
-    } catch (const std::system_error &) {
-      // fewer helpers
-    }
-  }
   // f(part, parts) for every part, the caller's part 0 included
   void run(int parts, const std::function<void(int, int)> &f) {
+    if (parts > 1 && !started_) start();
     parts = std::min(parts, (int)th_.size() + 1);
     if (parts > 1) {
       std::lock_guard<std::mutex> l(m_);
@@ -105,6 +96,18 @@ class Team {
   }
 
  private:
+  // the first transfer that shares its bytes out starts the helpers
+  void start() {
+    started_ = true;
+    cpu_set_t set;
+    int cpus = kThreads;
+    if (sched_getaffinity(0, sizeof set, &set) == 0) cpus = CPU_COUNT(&set);
+    try {
+      for (int i = 1; i < std::min(kThreads, cpus); ++i) th_.emplace_back([this, i] { work(i); });
+    } catch (const std::system_error &) {
+      // fewer helpers
+    }
+  }
   void work(int me) {
     uint64_t seen = 0;
     for (;;) {
@@ -133,24 +136,36 @@ class Team {
   std::atomic<int> left_{0};
   const std::function<void(int, int)> *f_ = nullptr;
   int parts_ = 0;
-  bool quit_ = false;
+  bool quit_ = false, started_ = false;
 };
 
 struct Stage {
   int device = 0;
   hipStream_t s = nullptr;
   char *buf[kSlots] = {};
+  size_t room[kSlots] = {};
   hipEvent_t done[kSlots] = {};
   Team team;
   bool ok = false;
   Stage() {
-    if (hipGetDevice(&device) != hipSuccess || hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return;
-    for (int i = 0; i < kSlots; ++i)
-      if (hipHostMalloc((void **)&buf[i], kChunk, hipHostMallocDefault) != hipSuccess ||
-          hipEventCreateWithFlags(&done[i], hipEventDisableTiming) != hipSuccess)
-        return;
-    team.start();
-    ok = true;
+    ok = hipGetDevice(&device) == hipSuccess && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess;
+    for (int i = 0; i < kSlots && ok; ++i) ok = hipEventCreateWithFlags(&done[i], hipEventDisableTiming) == hipSuccess;
+  }
+  // Buffers for a transfer of `bytes`, no more than it fills: 32 MiB of locked
+  // pages take 10 ms to get, a small field moves in a fraction of that.  Called
+  // with the stream idle.
+  bool reserve(size_t bytes) {
+    for (int i = 0; i < kSlots && (size_t)i * kChunk < bytes; ++i) {
+      size_t want = (size_t)256 << 10;
+      while (want < std::min(kChunk, bytes - (size_t)i * kChunk)) want *= 2;
+      if (room[i] >= want) continue;
+      if (buf[i]) (void)hipHostFree(buf[i]);
+      buf[i] = nullptr;
+      room[i] = 0;
+      if (hipHostMalloc((void **)&buf[i], want, hipHostMallocDefault) != hipSuccess) return false;
+      room[i] = want;
+    }
+    return true;
   }
   ~Stage() {
     if (s) (void)hipStreamSynchronize(s);
@@ -238,6 +253,7 @@ struct HostField {
 // the device work of bytes [at, at + len) on the stage's stream.
 template <typename Bus>
 int through(Stage &st, const HostField &h, size_t bytes, bool out, Bus bus) {
+  if (!st.reserve(bytes)) return fail(GPE_ENOMEM, "staging buffers");
   const size_t n = (bytes + kChunk - 1) / kChunk;
   auto put = [&](size_t i) {
     const size_t at = i * kChunk;
