@@ -128,4 +128,21 @@ __global__ void __launch_bounds__(64 * NW) brick_kernel(const StageArgs D) {
                                        A.part_energy);
 }
 
+// Many simulations: the work table holds the bricks of every instance in
+// order; each XCD's workgroups walk one contiguous part of it (gridDim.x is a
+// multiple of 8).
+template <typename T, int R, int NW, int ZB, int KIND, bool COMP>
+__global__ void __launch_bounds__(64 * NW)
+    brick_kernel_batched(const StageArgs *__restrict__ insts, const WorkItem *__restrict__ work, int nwork,
+                         const int *__restrict__ active, double *pn, double *pe) {
+  const int xcd = blockIdx.x & 7, q8 = nwork >> 3, r8 = nwork & 7;
+  const int first = xcd * q8 + min(xcd, r8), end = first + q8 + (xcd < r8);
+  for (int w = first + (blockIdx.x >> 3); w < end; w += gridDim.x >> 3) {
+    const WorkItem it = work[w];
+    if (active[it.inst])
+      brick_tile<T, R, NW, ZB, KIND, COMP>(args_at<T>(insts + it.inst), it.tx, it.ty, it.z0, it.slot, pn, pe, nullptr);
+    __syncthreads();  // the next item reuses the LDS bricks
+  }
+}
+
 }  // namespace gpe

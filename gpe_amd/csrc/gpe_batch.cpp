@@ -10,10 +10,11 @@
 // groups' stages + control) is captured once in a hipGraph and replayed;
 // the graph is captured again only when the set of instances changes.
 //
-// Per-site arithmetic is the single-simulation kernels' (stage_tile), so an
-// instance's field does not depend on the batch it runs in; its reductions
-// use only its own partial slots, in a fixed order, so its dt sequence and
-// norm do not either.
+// Per-site arithmetic is the single-simulation kernels' (stage_tile,
+// brick_tile), so an instance's field does not depend on the batch it runs in,
+// though how a stage is swept does; its reductions use only its own partial
+// slots, in an order that its own size fixes, so its dt sequence and norm do
+// not either.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,6 +38,13 @@ constexpr int kBatchDefaultVid = 0;
 int default_vid(int prec, int k) { return variant_allowed(prec == GPE_FP64, k, kBatchDefaultVid) ? kBatchDefaultVid : kVidF64Ck; }
 constexpr int kDefaultZc = 32;
 constexpr int kMaxGrid = 2048;  // persistent workgroups per batched launch
+
+// How a kind of a group is swept: in bricks of some planes, or by the z march
+// with a tile variant and z chunk (by_instance: no longer than chunk_of its size).
+struct Sweep {
+  int planes, vid, zc;
+  bool by_instance;
+};
 
 // Stage kinds of one iteration of each scheme: [k0, k0 + nk).
 void scheme_kinds(int scheme, int *k0, int *nk) {
@@ -107,6 +115,7 @@ struct Group {
   int pvid[P_COUNT], pzc[P_COUNT];
   KindTable ptab[P_COUNT];
   std::vector<int> slots;  // instance slots in this group, ascending
+  long long sites = 0;     // their grids' sites
   int part_off = 0;        // first partial slot of this group's final stage
 };
 
@@ -313,12 +322,68 @@ StageArgs inst_args(const Inst &I, int kind, const gpe_step_state &st) {
   return A;
 }
 
+// How kind k of a group is swept.  A configuration that was set (by hand or by
+// the autotuner) stays; the default one is chosen here.
+//
+// The group's sites together decide whether the chip is short of work: then
+// the chain of planes a workgroup marches through sets the time, and bricks or
+// short chunks shorten it; with much work, reading fields once does (launch.h,
+// brick_planes).  The lines are where the sides cross (MI355X, us an
+// iteration, against the (4,4) tile in chunks of 32 planes everywhere, FP64
+// Cash-Karp (8,1)):
+//   FP32C, sites x fields read, bricks / (8,1) tiles of 16:
+//     64^3, RK4 2nd order: k1..k3 -194 / -136 of 288
+//     5.3 M sites (6 grids of 48..128), RK45: ck_2 -38 / -36 of 603,
+//       ck_3 -35 / -32, ck_4 -24 / -28, ck_5 -11 / -21
+//     10.5 M sites, RK4: k1 -45 / -29 of 399, k2 -15 / -26
+//     22.6 M sites, RK45: ck_3 +50 / -22 of 1705, (8,2) tiles of 16: -44
+//   FP64, bricks / (4,2) tiles of 16:
+//     1.4 M sites, RK45: ck_2 -34 / -15 of 377, ck_3 -26 / -23, ck_5 -10 / -16
+//     3.5 M sites: ck_1 -90 / -57 of 832, ck_2 -49 / -46, ck_3 -13 / -35
+//     22.6 M sites: ck_1 -138 / -164 of 2991, ck_2 +19 / -107, ck_4 +469 / +13
+//
+// The last stage's tiles sum the instance's norm, whose last bits must not
+// depend on its companions: its tile is one for all groups, and its chunks go by
+// the instance's own size.  FP32C (8,1), chunks of 8 or 16: RK45 -103 of 541 at
+// 64^3, -116 of 582 at 1.4 M sites, -120 of 1705 at 22.6 M; FP64 RK4 (8,2) in
+// 8s: -84 of 417 at 128^3, -3 of 1318 at 22.6 M.
+//
+// All together, a whole iteration before and after: one 64^3 grid, FP32C RK4,
+// 292 -> 35 us; 6 grids of 48..128, FP64 RK4, 656 -> 359; 24 grids of 32..128,
+// FP32C RK4, 650 -> 596, FP64 RK45 3400 -> 2740.
+Sweep sweep_of(const Group &G, int k) {
+  const bool fp64 = G.prec == GPE_FP64;
+  if (G.vid[k] != default_vid(G.prec, k) || G.zc[k] != kDefaultZc) return {0, G.vid[k], G.zc[k], false};
+  if (k == G.k0 + G.nk - 1) {
+    if (k == K_RK2_2 || (fp64 && k == K_EULER)) return {0, 3, 16, true};
+    if (!fp64) return {0, k == K_EULER ? 1 : 4, 16, true};
+    return k == K_CK_6 ? Sweep{0, kVidF64Ck, 32, true} : Sweep{0, 1, 8, false};
+  }
+  const int reads = stage_reads(k);
+  if (!fp64) {
+    if (G.sites * reads <= 16000000) return {2, 0, 0, false};
+    return {0, reads == 1 ? 0 : G.sites <= 12000000 ? 4 : 1, 16, false};
+  }
+  if (reads == 1 && G.sites <= 10000000) return {4, 0, 0, false};
+  if (G.sites * reads <= 5000000) return {2, 0, 0, false};
+  if (G.sites <= 8000000) return {0, reads <= 4 ? 3 : 4, 16, false};
+  if (k == K_RK4_2 || reads >= 4) return {0, default_vid(G.prec, k), kDefaultZc, false};
+  return {0, 3, 16, false};
+}
+
+// Planes per chunk of an instance of n sites.
+int chunk_of(const Sweep &w, long long n) {
+  if (!w.by_instance) return w.zc;
+  return n <= 64 * 64 * 64 ? 8 : n <= 96 * 96 * 96 ? std::min(w.zc, 16) : w.zc;
+}
+
 // Work table of one kind of a group: every tile of every instance, each
 // instance's partial slots contiguous in (z, y, x) tile order; the table
 // itself is ordered largest tile first so the persistent grid ends evenly.
 // Work table over output tiles of TX x TY sites (a stage kind: 64 x TY; a
-// fused pair: the (64-2R) x (TY-2R) interiors).
-void make_table(gpe_batch *b, const Group &G, int TX, int TY, int zc, std::vector<WorkItem> &out,
+// fused pair: the (64-2R) x (TY-2R) interiors) and chunks of w.  Bricks take
+// equal time and stay in order.
+void make_table(gpe_batch *b, const Group &G, int TX, int TY, const Sweep &w, std::vector<WorkItem> &out,
                 std::vector<int> *range, int part_off) {
   out.clear();
   int slotc = part_off;
@@ -326,21 +391,14 @@ void make_table(gpe_batch *b, const Group &G, int TX, int TY, int zc, std::vecto
   for (int s : G.slots) {
     const Inst &I = b->slot[s];
     const int nx = I.P.nx, ny = I.P.ny, nz = I.P.nz;
-    const int zcl = zc > 0 ? std::min(zc, nz) : nz;
+    const int zc = w.planes ? w.planes : chunk_of(w, (long long)nx * ny * nz), zcl = zc > 0 ? std::min(zc, nz) : nz;
     const int ntx = (nx + TX - 1) / TX, nty = (ny + TY - 1) / TY;
     const int beg = slotc;
     for (int z0 = 0; z0 < nz; z0 += zcl) {
       const int z1 = std::min(z0 + zcl, nz);
       for (int ty = 0; ty < nty; ++ty)
         for (int tx = 0; tx < ntx; ++tx) {
-          WorkItem w;
-          w.inst = s;
-          w.tx = tx;
-          w.ty = ty;
-          w.z0 = z0;
-          w.z1 = z1;
-          w.slot = slotc++;
-          out.push_back(w);
+          out.push_back(WorkItem{s, tx, ty, z0, z1, slotc++});
           const long long cx = std::min(TX, nx - TX * tx), cy = std::min(TY, ny - TY * ty);
           cost.push_back((long long)(cx * cy) * (z1 - z0 + 2 * G.R));
         }
@@ -350,6 +408,7 @@ void make_table(gpe_batch *b, const Group &G, int TX, int TY, int zc, std::vecto
       (*range)[2 * s + 1] = slotc;
     }
   }
+  if (w.planes) return;
   std::vector<int> ord(out.size());
   for (size_t i = 0; i < ord.size(); ++i) ord[i] = (int)i;
   std::stable_sort(ord.begin(), ord.end(), [&](int a, int c) { return cost[a] > cost[c]; });
@@ -358,9 +417,9 @@ void make_table(gpe_batch *b, const Group &G, int TX, int TY, int zc, std::vecto
   out.swap(sorted);
 }
 
-void kind_tiles(int vid, int *TX, int *TY) {
+void kind_tiles(const Sweep &w, int *TX, int *TY) {
   *TX = 64;
-  *TY = kTiles[vid].nw * kTiles[vid].p;
+  *TY = w.planes ? kBrickWaves : kTiles[w.vid].nw * kTiles[w.vid].p;
 }
 
 void pair_tiles(const Group &G, int vid, int *TX, int *TY) {
@@ -380,7 +439,7 @@ int upload_table(KindTable &T) {
   }
   if (n) GPE_HIPCHK(hipMemcpy(T.d, T.h.data(), sizeof(WorkItem) * (size_t)n, hipMemcpyHostToDevice));
   T.n = n;
-  T.grid = std::min(n, kMaxGrid);
+  T.grid = std::min((n + 7) & ~7, kMaxGrid);
   return GPE_OK;
 }
 
@@ -408,16 +467,18 @@ int rebuild(gpe_batch *b) {
     G.slots.clear();
     for (int s = 0; s < b->cap; ++s)
       if (b->slot[s].id >= 0 && b->slot[s].group == (int)(&G - &b->groups[0])) G.slots.push_back(s);
+    G.sites = 0;
+    for (int s : G.slots) G.sites += (long long)b->slot[s].P.nx * b->slot[s].P.ny * b->slot[s].P.nz;
     G.part_off = part;
     for (const Unit &u : units_of(G)) {
       int TX, TY;
       KindTable &T = u.pair >= 0 ? G.ptab[u.pair] : G.tab[u.kind];
+      const Sweep w = u.pair >= 0 ? Sweep{0, 0, G.pzc[u.pair], false} : sweep_of(G, u.kind);
       if (u.pair >= 0)
         pair_tiles(G, G.pvid[u.pair], &TX, &TY);
       else
-        kind_tiles(G.vid[u.kind], &TX, &TY);
-      make_table(b, G, TX, TY, u.pair >= 0 ? G.pzc[u.pair] : G.zc[u.kind], T.h, u.final_ ? &range : nullptr,
-                 part);
+        kind_tiles(w, &TX, &TY);
+      make_table(b, G, TX, TY, w, T.h, u.final_ ? &range : nullptr, part);
       if ((rc = upload_table(T))) return rc;
       if (u.final_) part += (int)T.h.size();
     }
@@ -427,6 +488,13 @@ int rebuild(gpe_batch *b) {
   drop_graph(b);
   b->dirty = false;
   return GPE_OK;
+}
+
+hipError_t launch_sweep(const Group &G, int k, const Sweep &w, const BatchLaunch &L, hipStream_t s) {
+  const int pb = G.prec == GPE_FP64 ? 16 : 8;
+  const bool comp = G.prec == GPE_FP32C;
+  return w.planes ? launch_brick_batched(pb, w.planes, k, G.R, comp, L, s)
+                  : launch_stage_batched(pb, w.vid, k, G.R, comp, L, s);
 }
 
 // One iteration: every group's stages, then the per-instance control.
@@ -468,7 +536,7 @@ int enqueue_iteration(gpe_batch *b, bool fork) {
         L.pn = u.final_ ? b->d_pn : nullptr;
         L.pe = u.final_ ? b->d_pe : nullptr;
         L.grid = T.grid;
-        e = launch_stage_batched(G.prec == GPE_FP64 ? 16 : 8, G.vid[k], k, G.R, G.prec == GPE_FP32C, L, s);
+        e = launch_sweep(G, k, sweep_of(G, k), L, s);
       }
       if (e != hipSuccess) return fail(GPE_EHIP, "batched stage launch: %s", hipGetErrorString(e));
     }
@@ -919,7 +987,7 @@ int gpe_batch_tune_get(gpe_batch *b, int32_t precision, int32_t order, int32_t s
 // Time every tile variant and z-chunk for each stage kind of every group
 // over the current instances (reps launches each, stage kernels only: the
 // control kernel does not run, so no state is committed) and keep the
-// fastest.
+// fastest (the default configuration is timed as sweep_of sweeps it).
 int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
   if (!b) return fail(GPE_EINVAL, "batch is NULL");
   if (reps < 1) reps = 1;
@@ -937,14 +1005,18 @@ int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
     for (int k = G.k0; k < G.k0 + G.nk; ++k) {
       const bool fin = k == G.k0 + G.nk - 1;
       float best = 1e30f;
-      int bv = G.vid[k], bz = G.zc[k];
+      const int v0 = G.vid[k], z0 = G.zc[k];
+      int bv = v0, bz = z0;
       KindTable T;
       for (int v = 0; v < N_TILE_VARIANTS; ++v)
         for (int z : zcs) {
           if (!variant_allowed(G.prec == GPE_FP64, k, v)) continue;
           int TX, TY;
-          kind_tiles(v, &TX, &TY);
-          make_table(b, G, TX, TY, z, T.h, nullptr, 0);
+          G.vid[k] = v;
+          G.zc[k] = z;
+          const Sweep w = sweep_of(G, k);
+          kind_tiles(w, &TX, &TY);
+          make_table(b, G, TX, TY, w, T.h, nullptr, 0);
           if ((rc = upload_table(T)) || (rc = ensure_partials(b, T.n))) break;
           BatchLaunch L;
           L.insts = b->d_args + (size_t)k * b->cap;
@@ -954,11 +1026,9 @@ int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
           L.pn = fin ? b->d_pn : nullptr;
           L.pe = fin ? b->d_pe : nullptr;
           L.grid = T.grid;
-          const int pb = G.prec == GPE_FP64 ? 16 : 8;
-          const bool comp = G.prec == GPE_FP32C;
-          hipError_t e = launch_stage_batched(pb, v, k, G.R, comp, L, b->stream);  // warm
+          hipError_t e = launch_sweep(G, k, w, L, b->stream);  // warm
           e = e != hipSuccess ? e : hipEventRecord(e0, b->stream);
-          for (int r = 0; r < reps && e == hipSuccess; ++r) e = launch_stage_batched(pb, v, k, G.R, comp, L, b->stream);
+          for (int r = 0; r < reps && e == hipSuccess; ++r) e = launch_sweep(G, k, w, L, b->stream);
           e = e != hipSuccess ? e : hipEventRecord(e1, b->stream);
           e = e != hipSuccess ? e : hipEventSynchronize(e1);
           if (e != hipSuccess) {
@@ -974,9 +1044,9 @@ int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
           }
         }
       if (T.d) (void)hipFree(T.d);
+      G.vid[k] = rc ? v0 : bv;
+      G.zc[k] = rc ? z0 : bz;
       if (rc) break;
-      G.vid[k] = bv;
-      G.zc[k] = bz;
       kbest[k] = best;
     }
     if (rc) break;
@@ -993,7 +1063,7 @@ int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
         for (int z : {0, 32, 64}) {
           int TX, TY;
           pair_tiles(G, v, &TX, &TY);
-          make_table(b, G, TX, TY, z, T.h, nullptr, 0);
+          make_table(b, G, TX, TY, Sweep{0, 0, z, false}, T.h, nullptr, 0);
           if ((rc = upload_table(T)) || (rc = ensure_partials(b, T.n))) break;
           PairBatchLaunch L;
           L.instA = b->d_args + (size_t)k * b->cap;

@@ -146,6 +146,14 @@ struct BatchLaunch {
 };
 hipError_t launch_stage_batched(int prec_bytes, int vid, int kind, int radius, bool comp, const BatchLaunch &B,
                                 hipStream_t s);
+// B.grid: a multiple of 8
+hipError_t launch_brick_batched_f64(int planes, int kind, int radius, bool comp, const BatchLaunch &B, hipStream_t s);
+hipError_t launch_brick_batched_f32(int planes, int kind, int radius, bool comp, const BatchLaunch &B, hipStream_t s);
+inline hipError_t launch_brick_batched(int prec_bytes, int planes, int kind, int radius, bool comp,
+                                       const BatchLaunch &B, hipStream_t s) {
+  return prec_bytes == 16 ? launch_brick_batched_f64(planes, kind, radius, comp, B, s)
+                          : launch_brick_batched_f32(planes, kind, radius, comp, B, s);
+}
 struct PairBatchLaunch {
   const StageArgs *instA, *instB;  // stage A's / B's StageArgs of every instance slot
   const WorkItem *work;
