@@ -39,9 +39,9 @@ int default_vid(int prec, int k) { return variant_allowed(prec == GPE_FP64, k, k
 constexpr int kDefaultZc = 32;
 constexpr int kMaxGrid = 2048;  // persistent workgroups per batched launch
 
-// How a kind of a group is swept: in bricks of some planes, or by the z march
-// with a tile variant and z chunk (by_instance: no longer than chunk_of its size).
-struct Sweep {
+// How a kind of a group is swept (by_instance: chunks no longer than chunk_of
+// the instance's size).
+struct GroupSweep {
   int planes, vid, zc;
   bool by_instance;
 };
@@ -351,13 +351,13 @@ StageArgs inst_args(const Inst &I, int kind, const gpe_step_state &st) {
 // All together, a whole iteration before and after: one 64^3 grid, FP32C RK4,
 // 292 -> 35 us; 6 grids of 48..128, FP64 RK4, 656 -> 359; 24 grids of 32..128,
 // FP32C RK4, 650 -> 596, FP64 RK45 3400 -> 2740.
-Sweep sweep_of(const Group &G, int k) {
+GroupSweep sweep_of(const Group &G, int k) {
   const bool fp64 = G.prec == GPE_FP64;
   if (G.vid[k] != default_vid(G.prec, k) || G.zc[k] != kDefaultZc) return {0, G.vid[k], G.zc[k], false};
   if (k == G.k0 + G.nk - 1) {
     if (k == K_RK2_2 || (fp64 && k == K_EULER)) return {0, 3, 16, true};
     if (!fp64) return {0, k == K_EULER ? 1 : 4, 16, true};
-    return k == K_CK_6 ? Sweep{0, kVidF64Ck, 32, true} : Sweep{0, 1, 8, false};
+    return k == K_CK_6 ? GroupSweep{0, kVidF64Ck, 32, true} : GroupSweep{0, 1, 8, false};
   }
   const int reads = stage_reads(k);
   if (!fp64) {
@@ -372,7 +372,7 @@ Sweep sweep_of(const Group &G, int k) {
 }
 
 // Planes per chunk of an instance of n sites.
-int chunk_of(const Sweep &w, long long n) {
+int chunk_of(const GroupSweep &w, long long n) {
   if (!w.by_instance) return w.zc;
   return n <= 64 * 64 * 64 ? 8 : n <= 96 * 96 * 96 ? std::min(w.zc, 16) : w.zc;
 }
@@ -383,7 +383,7 @@ int chunk_of(const Sweep &w, long long n) {
 // Work table over output tiles of TX x TY sites (a stage kind: 64 x TY; a
 // fused pair: the (64-2R) x (TY-2R) interiors) and chunks of w.  Bricks take
 // equal time and stay in order.
-void make_table(gpe_batch *b, const Group &G, int TX, int TY, const Sweep &w, std::vector<WorkItem> &out,
+void make_table(gpe_batch *b, const Group &G, int TX, int TY, const GroupSweep &w, std::vector<WorkItem> &out,
                 std::vector<int> *range, int part_off) {
   out.clear();
   int slotc = part_off;
@@ -417,7 +417,7 @@ void make_table(gpe_batch *b, const Group &G, int TX, int TY, const Sweep &w, st
   out.swap(sorted);
 }
 
-void kind_tiles(const Sweep &w, int *TX, int *TY) {
+void kind_tiles(const GroupSweep &w, int *TX, int *TY) {
   *TX = 64;
   *TY = w.planes ? kBrickWaves : kTiles[w.vid].nw * kTiles[w.vid].p;
 }
@@ -473,7 +473,7 @@ int rebuild(gpe_batch *b) {
     for (const Unit &u : units_of(G)) {
       int TX, TY;
       KindTable &T = u.pair >= 0 ? G.ptab[u.pair] : G.tab[u.kind];
-      const Sweep w = u.pair >= 0 ? Sweep{0, 0, G.pzc[u.pair], false} : sweep_of(G, u.kind);
+      const GroupSweep w = u.pair >= 0 ? GroupSweep{0, 0, G.pzc[u.pair], false} : sweep_of(G, u.kind);
       if (u.pair >= 0)
         pair_tiles(G, G.pvid[u.pair], &TX, &TY);
       else
@@ -490,7 +490,7 @@ int rebuild(gpe_batch *b) {
   return GPE_OK;
 }
 
-hipError_t launch_sweep(const Group &G, int k, const Sweep &w, const BatchLaunch &L, hipStream_t s) {
+hipError_t launch_sweep(const Group &G, int k, const GroupSweep &w, const BatchLaunch &L, hipStream_t s) {
   const int pb = G.prec == GPE_FP64 ? 16 : 8;
   const bool comp = G.prec == GPE_FP32C;
   return w.planes ? launch_brick_batched(pb, w.planes, k, G.R, comp, L, s)
@@ -1014,7 +1014,7 @@ int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
           int TX, TY;
           G.vid[k] = v;
           G.zc[k] = z;
-          const Sweep w = sweep_of(G, k);
+          const GroupSweep w = sweep_of(G, k);
           kind_tiles(w, &TX, &TY);
           make_table(b, G, TX, TY, w, T.h, nullptr, 0);
           if ((rc = upload_table(T)) || (rc = ensure_partials(b, T.n))) break;
@@ -1063,7 +1063,7 @@ int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
         for (int z : {0, 32, 64}) {
           int TX, TY;
           pair_tiles(G, v, &TX, &TY);
-          make_table(b, G, TX, TY, Sweep{0, 0, z, false}, T.h, nullptr, 0);
+          make_table(b, G, TX, TY, GroupSweep{0, 0, z, false}, T.h, nullptr, 0);
           if ((rc = upload_table(T)) || (rc = ensure_partials(b, T.n))) break;
           PairBatchLaunch L;
           L.instA = b->d_args + (size_t)k * b->cap;

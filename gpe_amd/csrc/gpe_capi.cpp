@@ -139,6 +139,7 @@ struct gpe_ctx {
   std::vector<Ev> pending;
   std::vector<hipEvent_t> pool;
   int64_t prof_n[GPE_PROF_KINDS] = {};
+  int resident[K_COUNT] = {};  // workgroups of a kind's automatic march that a CU holds (0: not asked yet)
   DiagWork diag;  // lists of the vortex diagnostics
   // FFT-side diagnostics: a complex128 field and small scratch (on demand)
   void *spec = nullptr, *spec_aux = nullptr;
@@ -149,15 +150,26 @@ namespace {
 
 int grid_for_v(gpe_ctx *c, int vid, int zc, StageArgs &A) { return stage_grid(c->P.nx, c->P.ny, c->P.nz, vid, zc, A); }
 
-// Planes per brick of a kind's sweep, 0 for the z march: bricks are the
-// automatic configuration's choice (default tile, automatic z-chunk) only.
-int bricks_of(const gpe_ctx *c, int kind) {
+// How a kind is swept.  The default tile with an automatic z-chunk is the
+// automatic configuration: bricks or a tile and chunk chosen for the grid
+// (launch.h); every other one is taken as it is.
+Sweep sweep_of(gpe_ctx *c, int kind) {
   const bool fp64 = c->prec == GPE_FP64;
-  if (c->zc[kind] != 0 || c->vid[kind] != default_vid(fp64, kind)) return 0;
-  return brick_planes(fp64, kind, c->P.nx, c->P.ny, c->P.nz);
+  if (c->zc[kind] != 0 || c->vid[kind] != default_vid(fp64, kind)) return {0, c->vid[kind], c->zc[kind]};
+  const int nx = c->P.nx, ny = c->P.ny, nz = c->P.nz;
+  if (const int planes = brick_planes(fp64, kind, c->R, nx, ny, nz)) return {planes, 0, 0};
+  Sweep w{0, march_vid(fp64, kind, c->R, (long long)nx * ny * nz), 0};
+  if (kind == K_ENERGY) return w;
+  int &resident = c->resident[kind];
+  if (!resident && launch_stage((int)c->esz, w.vid, kind, c->R, c->comp, StageArgs{}, c->stream, &resident) != hipSuccess)
+    resident = 1;
+  w.zc = march_chunk(nx, ny, nz, w.vid, c->R, resident);
+  return w;
 }
 
-int grid_for(gpe_ctx *c, int kind, StageArgs &A) { return grid_for_v(c, c->vid[kind], c->zc[kind], A); }
+int grid_for(gpe_ctx *c, const Sweep &w, StageArgs &A) {
+  return w.planes ? brick_grid(c->P.nx, c->P.ny, c->P.nz, w.planes, A) : grid_for_v(c, w.vid, w.zc, A);
+}
 
 // Grid of a fused pair: tiles step by the (64-2R) x (TY-2R) interiors; the
 // z-chunks are long (each chunk primes 2R extra planes of stage A).
@@ -207,11 +219,8 @@ void prof_drain(gpe_ctx *c) {
 
 int run_kind(gpe_ctx *c, int kind, StageArgs &A) {
   Range range(kind_name(kind));
-  const int bricks = bricks_of(c, kind);
-  if (bricks)
-    brick_grid(c->P.nx, c->P.ny, c->P.nz, bricks, A);
-  else
-    grid_for(c, kind, A);
+  const Sweep w = sweep_of(c, kind);
+  grid_for(c, w, A);
   if ((kind_final(kind) || kind == K_ENERGY) && A.nblocks > c->part_cap)
     return fail(GPE_EINVAL, "internal: %d workgroups exceed partial buffer", A.nblocks);
   hipEvent_t ea = nullptr, eb = nullptr;
@@ -220,8 +229,8 @@ int run_kind(gpe_ctx *c, int kind, StageArgs &A) {
     eb = take_event(c);
     if (ea) (void)hipEventRecord(ea, c->stream);
   }
-  hipError_t e = bricks ? launch_brick((int)c->esz, bricks, kind, c->R, c->comp, A, c->stream)
-                        : launch_stage((int)c->esz, c->vid[kind], kind, c->R, c->comp, A, c->stream);
+  hipError_t e = w.planes ? launch_brick((int)c->esz, w.planes, kind, c->R, c->comp, A, c->stream)
+                          : launch_stage((int)c->esz, w.vid, kind, c->R, c->comp, A, c->stream);
   if (e != hipSuccess) return fail(GPE_EHIP, "stage %s launch: %s", kind_name(kind), hipGetErrorString(e));
   if (c->prof && ea && eb) {
     (void)hipEventRecord(eb, c->stream);
@@ -651,7 +660,8 @@ int gpe_ctx_create(const gpe_params *params, gpe_ctx **out) {
     }
     for (int kk = 0; kk < K_COUNT; ++kk) {
       StageArgs tmp{};
-      const int b = kind_final(kk) || kk == K_ENERGY ? bricks_of(c, kk) : 0;
+      const bool sums = kind_final(kk) || kk == K_ENERGY;
+      const int b = sums ? brick_planes(c->prec == GPE_FP64, kk, c->R, c->P.nx, c->P.ny, c->P.nz) : 0;
       if (b) cap = std::max(cap, brick_grid(c->P.nx, c->P.ny, c->P.nz, b, tmp));
     }
     if (cap < PW_BLOCKS) cap = PW_BLOCKS;

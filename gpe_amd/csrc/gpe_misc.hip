@@ -7,22 +7,22 @@
 namespace gpe {
 
 hipError_t launch_stage(int prec_bytes, int vid, int kind, int radius, bool comp, const StageArgs &A,
-                        hipStream_t s) {
+                        hipStream_t s, int *resident) {
   if (prec_bytes == 16) {
     switch (vid) {
-      case 0: return launch_stage_f64_v0(kind, radius, comp, A, s);
-      case 1: return launch_stage_f64_v1(kind, radius, comp, A, s);
-      case 2: return launch_stage_f64_v2(kind, radius, comp, A, s);
-      case 3: return launch_stage_f64_v3(kind, radius, comp, A, s);
-      case 4: return launch_stage_f64_v4(kind, radius, comp, A, s);
+      case 0: return launch_stage_f64_v0(kind, radius, comp, A, s, resident);
+      case 1: return launch_stage_f64_v1(kind, radius, comp, A, s, resident);
+      case 2: return launch_stage_f64_v2(kind, radius, comp, A, s, resident);
+      case 3: return launch_stage_f64_v3(kind, radius, comp, A, s, resident);
+      case 4: return launch_stage_f64_v4(kind, radius, comp, A, s, resident);
     }
   } else {
     switch (vid) {
-      case 0: return launch_stage_f32_v0(kind, radius, comp, A, s);
-      case 1: return launch_stage_f32_v1(kind, radius, comp, A, s);
-      case 2: return launch_stage_f32_v2(kind, radius, comp, A, s);
-      case 3: return launch_stage_f32_v3(kind, radius, comp, A, s);
-      case 4: return launch_stage_f32_v4(kind, radius, comp, A, s);
+      case 0: return launch_stage_f32_v0(kind, radius, comp, A, s, resident);
+      case 1: return launch_stage_f32_v1(kind, radius, comp, A, s, resident);
+      case 2: return launch_stage_f32_v2(kind, radius, comp, A, s, resident);
+      case 3: return launch_stage_f32_v3(kind, radius, comp, A, s, resident);
+      case 4: return launch_stage_f32_v4(kind, radius, comp, A, s, resident);
     }
   }
   return hipErrorInvalidValue;

@@ -68,7 +68,7 @@ extern "C" int gpe_energy_noalloc(const gpe_params *params, const void *psi, dou
   // the launch configuration of a new context (gpe_ctx_create), so the
   // partial sums and their order equal gpe_sim_energy's
   const int vid = kDefaultVid;
-  const int bricks = brick_planes(prec == GPE_FP64, K_ENERGY, params->nx, params->ny, params->nz);
+  const int bricks = brick_planes(prec == GPE_FP64, K_ENERGY, params->order / 2, params->nx, params->ny, params->nz);
   const int nb = bricks ? brick_grid(params->nx, params->ny, params->nz, bricks, A)
                         : stage_grid(params->nx, params->ny, params->nz, vid, 0, A);
   if (nb > kMaxPartials)

@@ -27,7 +27,10 @@ namespace {
 constexpr Tile kT = kTiles[GPE_VID];
 
 template <int R, int KIND, bool COMP>
-hipError_t launch_one(const StageArgs &A, hipStream_t s) {
+hipError_t launch_one(const StageArgs &A, hipStream_t s, int *resident) {
+  if (resident)
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        resident, (const void *)stage_kernel<GPE_REAL, R, kT.nw, kT.p, KIND, COMP>, 64 * kT.nw, 0);
   hipLaunchKernelGGL((stage_kernel<GPE_REAL, R, kT.nw, kT.p, KIND, COMP>), dim3(A.nblocks), dim3(64 * kT.nw), 0, s,
                      A);
   return hipGetLastError();
@@ -61,36 +64,37 @@ hipError_t launch_rb(int kind, const BatchLaunch &B, hipStream_t s) {
 }
 
 template <int R, bool COMP>
-hipError_t launch_r(int kind, const StageArgs &A, hipStream_t s) {
+hipError_t launch_r(int kind, const StageArgs &A, hipStream_t s, int *resident) {
   switch (kind) {
-    case K_RHS: return launch_one<R, K_RHS, false>(A, s);
-    case K_EULER: return launch_one<R, K_EULER, COMP>(A, s);
-    case K_RK2_1: return launch_one<R, K_RK2_1, false>(A, s);
-    case K_RK2_2: return launch_one<R, K_RK2_2, COMP>(A, s);
-    case K_RK4_1: return launch_one<R, K_RK4_1, false>(A, s);
-    case K_RK4_2: return launch_one<R, K_RK4_2, false>(A, s);
-    case K_RK4_3: return launch_one<R, K_RK4_3, false>(A, s);
-    case K_RK4_4: return launch_one<R, K_RK4_4, COMP>(A, s);
-    case K_CK_1: return launch_one<R, K_CK_1, COMP>(A, s);
-    case K_CK_2: return launch_one<R, K_CK_2, COMP>(A, s);
-    case K_CK_3: return launch_one<R, K_CK_3, COMP>(A, s);
-    case K_CK_4: return launch_one<R, K_CK_4, COMP>(A, s);
-    case K_CK_5: return launch_one<R, K_CK_5, COMP>(A, s);
-    case K_CK_6: return launch_one<R, K_CK_6, COMP>(A, s);
-    case K_ENERGY: return launch_one<R, K_ENERGY, false>(A, s);
+    case K_RHS: return launch_one<R, K_RHS, false>(A, s, resident);
+    case K_EULER: return launch_one<R, K_EULER, COMP>(A, s, resident);
+    case K_RK2_1: return launch_one<R, K_RK2_1, false>(A, s, resident);
+    case K_RK2_2: return launch_one<R, K_RK2_2, COMP>(A, s, resident);
+    case K_RK4_1: return launch_one<R, K_RK4_1, false>(A, s, resident);
+    case K_RK4_2: return launch_one<R, K_RK4_2, false>(A, s, resident);
+    case K_RK4_3: return launch_one<R, K_RK4_3, false>(A, s, resident);
+    case K_RK4_4: return launch_one<R, K_RK4_4, COMP>(A, s, resident);
+    case K_CK_1: return launch_one<R, K_CK_1, COMP>(A, s, resident);
+    case K_CK_2: return launch_one<R, K_CK_2, COMP>(A, s, resident);
+    case K_CK_3: return launch_one<R, K_CK_3, COMP>(A, s, resident);
+    case K_CK_4: return launch_one<R, K_CK_4, COMP>(A, s, resident);
+    case K_CK_5: return launch_one<R, K_CK_5, COMP>(A, s, resident);
+    case K_CK_6: return launch_one<R, K_CK_6, COMP>(A, s, resident);
+    case K_ENERGY: return launch_one<R, K_ENERGY, false>(A, s, resident);
     default: return hipErrorInvalidValue;
   }
 }
 }  // namespace
 
-hipError_t GPE_FN2(GPE_PNAME, GPE_VID)(int kind, int radius, bool comp, const StageArgs &A, hipStream_t s) {
+hipError_t GPE_FN2(GPE_PNAME, GPE_VID)(int kind, int radius, bool comp, const StageArgs &A, hipStream_t s,
+                                        int *resident) {
 #ifdef GPE_F64
   (void)comp;
-  if (radius == 1) return launch_r<1, false>(kind, A, s);
-  if (radius == 2) return launch_r<2, false>(kind, A, s);
+  if (radius == 1) return launch_r<1, false>(kind, A, s, resident);
+  if (radius == 2) return launch_r<2, false>(kind, A, s, resident);
 #else
-  if (radius == 1) return comp ? launch_r<1, true>(kind, A, s) : launch_r<1, false>(kind, A, s);
-  if (radius == 2) return comp ? launch_r<2, true>(kind, A, s) : launch_r<2, false>(kind, A, s);
+  if (radius == 1) return comp ? launch_r<1, true>(kind, A, s, resident) : launch_r<1, false>(kind, A, s, resident);
+  if (radius == 2) return comp ? launch_r<2, true>(kind, A, s, resident) : launch_r<2, false>(kind, A, s, resident);
 #endif
   return hipErrorInvalidValue;
 }

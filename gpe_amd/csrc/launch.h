@@ -70,6 +70,12 @@ constexpr int stage_reads(int kind) {
                                                                : 1;
 }
 
+// A single simulation's sweep: bricks of some planes, or (planes 0) the march
+// with a tile variant and z-chunk.
+struct Sweep {
+  int planes, vid, zc;
+};
+
 // Brick sweeps (brick.hpp): kBrickWaves rows and 2 or 4 planes per workgroup.
 constexpr int kBrickWaves = 8;
 inline int brick_grid(int nx, int ny, int nz, int planes, StageArgs &A) {
@@ -95,13 +101,78 @@ inline int brick_grid(int nx, int ny, int nz, int planes, StageArgs &A) {
 // take bricks of 4 planes beyond that: at 256^3 rk4_1 185 -> 135, rk4_2
 // 256 -> 231 (2nd order), ck_1 323 -> 206, ck_2 256 -> 226; at 384^3 rk4_1
 // 615 -> 425, but rk4_2 782 -> 866.
-inline int brick_planes(bool fp64, int kind, int nx, int ny, int nz) {
+inline int brick_planes(bool fp64, int kind, int radius, int nx, int ny, int nz) {
   const long long n = (long long)nx * ny * nz;
   const int reads = stage_reads(kind);
   StageArgs A;
-  if (n * reads <= (fp64 ? 5000000 : 8000000)) return brick_grid(nx, ny, nz, 2, A) <= 65536 ? 2 : 0;
-  if (fp64 && kind != K_ENERGY && (reads == 1 || (reads == 2 && n <= 20000000))) return 4;
-  return 0;
+  // 4th order in FP32, one field: the march with (4,2) tiles is ahead earlier
+  // (ck_1 at 2.4 M sites 24 -> 21, 225^3 45 -> 35)
+  const long long most = fp64 ? 5000000 : reads == 1 && radius == 2 && kind != K_ENERGY ? 2000000 : 8000000;
+  if (n * reads <= most) return brick_grid(nx, ny, nz, 2, A) <= 65536 ? 2 : 0;
+  if (!fp64 || kind == K_ENERGY || reads > 2) return 0;
+  if (kind == K_CK_1) return 4;
+  // as above for 4th-order kinds that the march with (4,2) tiles serves well:
+  // rk4_1 at 192^3 81 -> 73, 320^3 322 -> 264, rk4_3 103 -> 85 and 445 -> 338,
+  // ck_2 101 -> 86 and 547 -> 350
+  const bool early = radius == 2 && kind != K_RK4_2 && kind != K_RK2_2;
+  if (reads == 1) return early && n > 6000000 ? 0 : 4;
+  // rk4_2's march wants whole tiles (256^3 270 -> 219, but 257 x 255 x 258 291 -> 329)
+  const bool whole = radius == 2 && kind == K_RK4_2 && nx % 64 == 0;
+  return n <= (early || whole ? 6000000 : 20000000) ? 4 : 0;
+}
+
+// Tile variant of the z march where a kind's configuration is automatic: the
+// fastest of the five over grids of 0.5 .. 134 M sites, each with chunks of
+// march_chunk.  FP64 kinds are bound by instructions and by the latency of a
+// plane, so the variants with the fewest registers per lane and more
+// workgroups win ((4,2) against (8,2), 4th order: 256^3 rk4_4 283 -> 229 us,
+// 512^3 rk4_3 1590 -> 1300, ck_2 against (8,1) 2060 -> 1340; (16,1) for ck_3
+// and ck_4, 256^3 319 -> 261); the FP32 ones keep (8,2) but for those that
+// store little or read one field (rk4_1 at 256^3 82 -> 65, rk4_2 157 -> 118).
+inline int march_vid(bool fp64, int kind, int radius, long long n) {
+  const bool r2 = radius == 2;
+  if (kind == K_ENERGY) return kDefaultVid;
+  if (!fp64) {
+    if (kind == K_EULER) return 1;
+    if (stage_reads(kind) == 1) return n < 50000000 ? 3 : 0;
+    if (kind == K_RK4_2 && r2) return n < 5000000 ? 3 : 0;
+    return kind == K_RK2_2 && r2 ? 4 : 1;
+  }
+  switch (kind) {
+    case K_RK4_2: return r2 ? 0 : 3;
+    case K_RK2_2: return r2 ? 1 : 3;
+    case K_CK_3:
+    case K_CK_4: return r2 ? 2 : 3;
+    case K_CK_5: return r2 ? 4 : 3;
+    case K_CK_6: return 4;
+    default: return 3;
+  }
+}
+
+// Planes per chunk of the march, automatic: a CU holds `resident` of the
+// kind's workgroups, so a sweep takes ceil(workgroups / (CUs x resident))
+// rounds of zc + 2R planes each, and the chunk with the smallest product wins:
+// long enough that few planes are read twice, and with no round that is nearly
+// empty (FP64 ck_6 at 192^3: chunks of 8, 16, 32, 64 planes take 7, 4, 2, 1
+// rounds and 250, 243, 223, 208 us).  Over grids of 0.5 .. 134 M sites, every
+// kind and tile, it comes within 1 .. 2 % of the best of 8, 16, 32 and 64.
+constexpr int kCUs = 256;
+inline int march_chunk(int nx, int ny, int nz, int vid, int radius, int resident) {
+  const Tile t = kTiles[vid];
+  const long long tiles2d = (long long)((nx + 63) / 64) * ((ny + t.nw * t.p - 1) / (t.nw * t.p));
+  const long long room = (long long)kCUs * (resident > 0 ? resident : 1);
+  int best = nz;
+  long long least = 0;
+  for (int n = 1; n == 1 || (nz + n - 1) / n >= 8; ++n) {
+    const int zc = (nz + n - 1) / n;
+    const long long groups = tiles2d * ((nz + zc - 1) / zc);
+    const long long cost = (groups + room - 1) / room * (zc + 2 * radius);
+    if (n == 1 || cost < least) {
+      least = cost;
+      best = zc;
+    }
+  }
+  return best;
 }
 hipError_t launch_brick_f64(int planes, int kind, int radius, bool comp, const StageArgs &A, hipStream_t s);
 hipError_t launch_brick_f32(int planes, int kind, int radius, bool comp, const StageArgs &A, hipStream_t s);
@@ -112,9 +183,10 @@ inline hipError_t launch_brick(int prec_bytes, int planes, int kind, int radius,
 }
 
 // Launch stage kernel `kind` (radius 1 or 2) over A.nblocks workgroups with
-// tile variant `vid`.  comp selects the compensated FP32 form.
+// tile variant `vid`.  comp selects the compensated FP32 form.  With resident,
+// nothing is launched: how many of its workgroups a CU holds at once.
 hipError_t launch_stage(int prec_bytes, int vid, int kind, int radius, bool comp, const StageArgs &A,
-                        hipStream_t s);
+                        hipStream_t s, int *resident = nullptr);
 
 // Fused stage pairs (fused.hpp): pair kinds P_RK4_12 .. P_CK_56 and their
 // tile variants.
@@ -197,7 +269,8 @@ hipError_t probe_bandwidth(size_t bytes, int reps, double *gbs);
 
 // per-variant entry points (one definition per translation unit)
 #define GPE_DECL_VARIANT(P, V) \
-  hipError_t launch_stage_##P##_v##V(int kind, int radius, bool comp, const StageArgs &A, hipStream_t s);
+  hipError_t launch_stage_##P##_v##V(int kind, int radius, bool comp, const StageArgs &A, hipStream_t s, \
+                                     int *resident);
 GPE_DECL_VARIANT(f64, 0)
 GPE_DECL_VARIANT(f64, 1)
 GPE_DECL_VARIANT(f64, 2)
