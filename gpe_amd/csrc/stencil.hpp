@@ -589,9 +589,11 @@ __device__ __forceinline__ void emit_site(Args<T> &A, const bool act, const size
             stc<T>(A.psi_out, s, nf);
             np = todbl(nf);
           }
-          // |scale|^2, or in the compensated form its term |psi|^2
+          // |scale|^2, or in the compensated form its term |psi|^2 (a negative
+          // time step takes the term dt |f| away: then every site is measured)
           const cx<T> sc = COMP ? F[0] : o[0];
-          lead = err_may_lead(err, sc.re * sc.re + sc.im * sc.im, sum.thr);
+          const T s2 = sc.re * sc.re + sc.im * sc.im;
+          lead = err_may_lead(err, COMP && !(A.sdtr >= 0.0) ? (T)0 : s2, sum.thr);
           sum.norm += wn * (np.re * np.re + np.im * np.im);
         }
       } else if constexpr (KI::final_) {
