@@ -224,8 +224,10 @@ __device__ __forceinline__ bool err_may_lead(cx<float> e, float s2, float thr) {
 }
 // The next thr of a wave whose lanes' largest values are m (NaN: ignored),
 // all lanes active.  A maximum over the lanes in single precision, by lane
-// shifts within the vector unit (rounding is inside the margin; a value
-// outside the single range gives a thr that decides nothing).
+// shifts within the vector unit: rounding is inside the margin where the value
+// and, in single precision, its square are normal; a smaller one (a subnormal
+// may round up by half of itself) gives a thr of 0 and a larger one infinity,
+// which decide nothing.
 template <typename T>
 __device__ __forceinline__ T err_lead(double m) {
   float x = fmaxf((float)m, 0.0f);
@@ -239,7 +241,9 @@ __device__ __forceinline__ T err_lead(double m) {
   x = fmaxf(x, shifted(std::integral_constant<int, 0x142>()));  // row_bcast:15, 31
   x = fmaxf(x, shifted(std::integral_constant<int, 0x143>()));
   x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
-  return (T)x * (T)x * (T)(1.0 - 0x1p-10);
+  const T t = (T)x * (T)x * (T)(1.0 - 0x1p-10);
+  constexpr T least = std::is_same<T, double>::value ? (T)0 : (T)0x1p-126f;
+  return x >= 0x1p-126f && t >= least ? t : (T)0;
 }
 
 // Index map for a ghost index i in [-R, n-1+R].
