@@ -3,7 +3,6 @@
 #pragma once
 #include <cmath>
 #include <cstdint>
-#include <cstdlib>
 
 #ifdef __HIPCC__
 #define GPE_DIVC_HD __host__ __device__ __forceinline__
@@ -23,11 +22,13 @@ namespace gpe {
 // advance", IEEE Trans. Computers 53, 2004), but for some d and zl on a few
 // numerators whose quotient lies next to the middle of two doubles.
 // make_divc enumerates those and takes a zh, zl for which every one rounds
-// as it should; 0.04% of random divisors have none, and their quotients
+// as it should; 0.08% of random divisors have none, and their quotients
 // differ in the last bit on a handful of the 2^53 numerators.
-// The constants carry powers of two that cancel: cs = c*2^K (no tiny
-// numerator loses bits in t*zl) and zh, zl a factor 2^-(e+K), so the final
-// * 2^-e costs nothing.
+// zh and zl carry the factor 2^-e, so the final * 2^-e costs nothing.
+// Numerators may be as large as for the division itself; the smallest are
+// 2^-900 for divisors from 2^-1022 to 2^100 (below, t*zl loses bits).  An
+// infinite numerator gives an infinity, but NaN where zl < 0 (3% of random
+// divisors: no zl >= 0 rounds every quotient).
 struct DivC {
   double cs, zh, zl;
 };
@@ -95,10 +96,10 @@ inline DivC make_divc(double s) {
       found = true;
     }
   }
-  const int K = std::abs(e) <= 512 ? 256 : 0;
-  d.cs = std::ldexp(c, K);
-  d.zh = std::ldexp(zh, -(e + K));
-  d.zl = std::ldexp(zl, -(e + K));
+  if (zl == 0.0) zl = 0x1p-200;  // d = 1: too small to count, but an infinity times it is one
+  d.cs = c;
+  d.zh = std::ldexp(zh, -e);
+  d.zl = std::ldexp(zl, -e);
   return d;
 }
 

@@ -81,3 +81,19 @@ def test_undefined_divisors_give_nan(shim):
     for s in (0.0, float("inf"), float("nan")):
         shim.divc(s, _p(a), 3, _p(got), _p(want))
         assert np.isnan(got).all()
+
+
+def test_numerators_to_the_end_of_the_range(shim):
+    # quotients of the largest numerators whose a*c does not overflow; by the
+    # package's own divisors also where it does, and of infinities
+    rng = np.random.default_rng(12)
+    own = [1.92, 12 * 0.4 ** 2, 0.4 ** 2, 12 * 0.25 ** 2, 12 * 0.5 ** 2, 0.25, 0.5, 1.0, 2.0, 4.0, 6.0, 3.0, 12 * 0.1]
+    with np.errstate(over="ignore"):
+        for s in own + [0.01, 1e-30, 1e30] + list(np.exp(rng.uniform(-8, 8, 200))):
+            a = np.concatenate([rng.standard_normal(4000) * 2.0 ** rng.integers(240, 1022, 4000),
+                                rng.uniform(-1, 1, 2000) * (1.79e308 if s in own else 0.89e308), [1e232],
+                                [1.7976931348623157e308, np.inf, -np.inf] if s in own else []])
+            got, want = np.empty_like(a), np.empty_like(a)
+            shim.divc(s, _p(a), len(a), _p(got), _p(want))
+            same = got == want
+            assert same.all(), (s, a[~same][:3], got[~same][:3], want[~same][:3])

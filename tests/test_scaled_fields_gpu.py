@@ -63,3 +63,21 @@ def test_rk45_steps(gpu, oracle, scale, shape):
             got, s = sim.download(), sim.state()
         assert np.array_equal(got, want)
         assert s["dt"].real == st.dt_re and s["errmax"] == st.errmax
+
+
+@pytest.mark.parametrize("scale", [1e-200, 1.0, 1e235, 1e300])
+def test_renormalise(gpu, scale):
+    # (sqrt(nn) psi) / sqrt(norm) as the reference divides a complex by a real:
+    # (a c) / c^2 * 2^-e with norm's root c 2^e
+    from gpe_amd.sim import Simulation
+    cfg = _cfg(nx=20, ny=12, nz=10)
+    psi = _field(cfg, scale)
+    print("[case] renormalise", scale, flush=True)
+    for norm in (1.92 ** 2, 0.0625, 702.0):
+        b = np.sqrt(norm)
+        e = np.floor(np.log2(b))
+        c = b * 2.0 ** -e
+        with Simulation(cfg, psi) as sim:
+            sim.renormalise(2.25, norm)
+            got = sim.download()
+        assert np.array_equal(got.view(np.float64), (1.5 * psi.view(np.float64) * c) / (c * c) * 2.0 ** -e)
