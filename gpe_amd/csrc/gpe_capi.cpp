@@ -122,7 +122,7 @@ struct gpe_ctx {
   gpe_step_state st{};
   StageArgs base{};
   // launch configuration per stage kind: tile variant (index into kTiles)
-  // and z-chunk length (0 = automatic)
+  // and z-chunk length (0: stage_grid's; kAutoChunk: the sweep is chosen)
   int vid[K_COUNT];
   int zc[K_COUNT];
   // fused stage pairs: on/off, tile variant and z-chunk per pair kind
@@ -150,16 +150,14 @@ namespace {
 
 int grid_for_v(gpe_ctx *c, int vid, int zc, StageArgs &A) { return stage_grid(c->P.nx, c->P.ny, c->P.nz, vid, zc, A); }
 
-// How a kind is swept.  The default tile with an automatic z-chunk is the
-// automatic configuration: bricks or a tile and chunk chosen for the grid
-// (launch.h); every other one is taken as it is.
+// How a kind is swept: as it was set, or (automatic) in bricks or by a tile and
+// chunk chosen for the grid (launch.h).
 Sweep sweep_of(gpe_ctx *c, int kind) {
+  if (c->zc[kind] != kAutoChunk) return {0, c->vid[kind], c->zc[kind]};
   const bool fp64 = c->prec == GPE_FP64;
-  if (c->zc[kind] != 0 || c->vid[kind] != default_vid(fp64, kind)) return {0, c->vid[kind], c->zc[kind]};
   const int nx = c->P.nx, ny = c->P.ny, nz = c->P.nz;
-  if (const int planes = brick_planes(fp64, kind, c->R, nx, ny, nz)) return {planes, 0, 0};
-  Sweep w{0, march_vid(fp64, kind, c->R, (long long)nx * ny * nz), 0};
-  if (kind == K_ENERGY) return w;
+  Sweep w{brick_planes(fp64, kind, c->R, nx, ny, nz), march_vid(fp64, kind, c->R, (long long)nx * ny * nz), 0};
+  if (w.planes || kind == K_ENERGY) return w;
   int &resident = c->resident[kind];
   if (!resident && launch_stage((int)c->esz, w.vid, kind, c->R, c->comp, StageArgs{}, c->stream, &resident) != hipSuccess)
     resident = 1;
@@ -629,11 +627,11 @@ int gpe_ctx_create(const gpe_params *params, gpe_ctx **out) {
   // the compensated form forms the rk45 error scale in the last stage
   if (params->scheme == GPE_RK45 && !c->comp && (rc = alloc_field(c, &c->scale))) goto bad;
   {
-    // default launch configuration; partial buffers sized for the largest
+    // automatic launch configuration; partial buffers sized for the largest
     // grid any variant and z-chunk can produce
     for (int kk = 0; kk < K_COUNT; ++kk) {
-      c->vid[kk] = default_vid(c->prec == GPE_FP64, kk);
-      c->zc[kk] = 0;
+      c->vid[kk] = kDefaultVid;
+      c->zc[kk] = kAutoChunk;
     }
     // every pair runs as its two stages until the autotuner (or
     // gpe_tune_set with a variant >= 0) finds the fused sweep faster: the
@@ -1110,9 +1108,9 @@ int gpe_tune_set(gpe_ctx *c, int32_t kind, int32_t variant, int32_t zchunk) {
   if (variant < 0 || variant >= N_TILE_VARIANTS) return fail(GPE_EINVAL, "variant out of range");
   if (!variant_allowed(c->prec == GPE_FP64, kind, variant))
     return fail(GPE_EINVAL, "FP64 Cash-Karp stages do not run tile variant %d", variant);
-  if (zchunk < 0) return fail(GPE_EINVAL, "zchunk < 0");
+  if (zchunk < 0 && !automatic_chunk(zchunk)) return fail(GPE_EINVAL, "zchunk < 0");
   c->vid[kind] = variant;
-  c->zc[kind] = zchunk;
+  c->zc[kind] = zchunk < 0 ? kAutoChunk : zchunk;
   return GPE_OK;
 }
 
@@ -1128,10 +1126,11 @@ int gpe_tune_get(gpe_ctx *c, int32_t kind, int32_t *variant, int32_t *zchunk, in
     return GPE_OK;
   }
   if (kind < 0 || kind >= K_COUNT) return fail(GPE_EINVAL, "kind out of range");
-  if (variant) *variant = c->vid[kind];
-  if (zchunk) *zchunk = c->zc[kind];
-  if (nw) *nw = kTiles[c->vid[kind]].nw;
-  if (rows) *rows = kTiles[c->vid[kind]].p;
+  const Sweep w = sweep_of(c, kind);
+  if (variant) *variant = w.vid;
+  if (zchunk) *zchunk = w.planes ? -w.planes : c->zc[kind];
+  if (nw) *nw = w.planes ? kBrickWaves : kTiles[w.vid].nw;
+  if (rows) *rows = w.planes ? 1 : kTiles[w.vid].p;
   return GPE_OK;
 }
 
@@ -1201,8 +1200,9 @@ int gpe_tune_load(gpe_ctx *c, const char *path, int32_t *applied) {
   return GPE_OK;
 }
 
-// Time every tile variant and a few z-chunk lengths of each stage kind of
-// the context's scheme on the resident field, keep the fastest.  Outputs go
+// Time the automatic sweep and every tile variant with a few z-chunk lengths of
+// each stage kind of the context's scheme on the resident field, keep the
+// fastest.  Outputs go
 // to the work fields (k, acc, next state), which every step rewrites before
 // reading, so the state is unchanged.
 int gpe_autotune(gpe_ctx *c, int32_t reps) {
@@ -1317,32 +1317,32 @@ int gpe_autotune(gpe_ctx *c, int32_t reps) {
     if (kind == K_RK4_3) { A.kin[0] = c->k[1]; A.kout = c->k[0]; }
     std::vector<int> zcs = {0, 16, 32, 64, 128, 256, 512};  // as for the pairs
     if (c->P.nz > 512) zcs.push_back(c->P.nz);
+    std::vector<std::pair<int, int>> trials = {{c->vid[kind], kAutoChunk}};
+    for (int v = 0; v < N_TILE_VARIANTS; ++v)
+      for (int zc : zcs)
+        if (variant_allowed(c->prec == GPE_FP64, kind, v) && zc <= c->P.nz) trials.push_back({v, zc});
     float best = 1e30f;
     int bv = c->vid[kind], bz = c->zc[kind];
-    for (int v = 0; v < N_TILE_VARIANTS && rc == GPE_OK; ++v) {
-      if (!variant_allowed(c->prec == GPE_FP64, kind, v)) continue;
-      for (int zc : zcs) {
-        if (zc > c->P.nz) continue;
-        c->vid[kind] = v;
-        c->zc[kind] = zc;
-        if ((rc = run_kind(c, kind, A))) break;  // warm
-        if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = fail(GPE_EHIP, "event"); break; }
-        for (int r = 0; r < reps && rc == GPE_OK; ++r) rc = run_kind(c, kind, A);
-        if (rc) break;
-        float ms = 0.f;
-        hipError_t he = hipEventRecord(e1, c->stream);
-        if (he == hipSuccess) he = hipEventSynchronize(e1);
-        if (he == hipSuccess) he = hipEventElapsedTime(&ms, e0, e1);
-        if (he != hipSuccess) {
-          // a failed trial must not be taken for the fastest
-          rc = fail(GPE_EHIP, "autotune timing: %s", hipGetErrorString(he));
-          break;
-        }
-        if (ms < best) {
-          best = ms;
-          bv = v;
-          bz = zc;
-        }
+    for (const auto &[v, zc] : trials) {
+      c->vid[kind] = v;
+      c->zc[kind] = zc;
+      if ((rc = run_kind(c, kind, A))) break;  // warm
+      if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = fail(GPE_EHIP, "event"); break; }
+      for (int r = 0; r < reps && rc == GPE_OK; ++r) rc = run_kind(c, kind, A);
+      if (rc) break;
+      float ms = 0.f;
+      hipError_t he = hipEventRecord(e1, c->stream);
+      if (he == hipSuccess) he = hipEventSynchronize(e1);
+      if (he == hipSuccess) he = hipEventElapsedTime(&ms, e0, e1);
+      if (he != hipSuccess) {
+        // a failed trial must not be taken for the fastest
+        rc = fail(GPE_EHIP, "autotune timing: %s", hipGetErrorString(he));
+        break;
+      }
+      if (ms < best) {
+        best = ms;
+        bv = v;
+        bz = zc;
       }
     }
     c->vid[kind] = bv;

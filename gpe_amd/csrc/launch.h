@@ -30,11 +30,9 @@ constexpr bool variant_allowed(bool fp64, int kind, int vid) {
   return vid >= 0 && vid < N_TILE_VARIANTS && !(fp64 && kind >= K_CK_1 && kind <= K_CK_6 && vid <= 1);
 }
 
-// Tile variant of a new context's stage kinds (the (8,2) tile), where allowed.
+// The (8,2) tile: the automatic march of the kinds that nothing else serves
+// better.
 constexpr int kDefaultVid = 1;
-constexpr int default_vid(bool fp64, int kind) {
-  return variant_allowed(fp64, kind, kDefaultVid) ? kDefaultVid : kVidF64Ck;
-}
 
 // Tiling of one stage sweep over an nx x ny x nz grid with tile variant vid
 // and z-chunk zc (0: automatic): sets A.ntx, A.nty, A.zc, A.nzc and
@@ -76,6 +74,11 @@ struct Sweep {
   int planes, vid, zc;
 };
 
+// The z-chunk of a kind in its automatic configuration, in which every kind
+// starts; one that was read (-planes for bricks) sets it too.
+constexpr int kAutoChunk = -1;
+constexpr bool automatic_chunk(int zc) { return zc == kAutoChunk || zc == -2 || zc == -4; }
+
 // Brick sweeps (brick.hpp): kBrickWaves rows and 2 or 4 planes per workgroup.
 constexpr int kBrickWaves = 8;
 inline int brick_grid(int nx, int ny, int nz, int planes, StageArgs &A) {
@@ -87,8 +90,8 @@ inline int brick_grid(int nx, int ny, int nz, int planes, StageArgs &A) {
   return A.nblocks;
 }
 
-// Planes per brick with which a kind in its automatic configuration (default
-// tile, automatic z-chunk) sweeps a grid, or 0 for the z march.  A brick reads
+// Planes per brick with which a kind in its automatic configuration sweeps a
+// grid, or 0 for the z march.  A brick reads
 // each of its fields about three times (2 planes, 4th order) where the march
 // reads them once, so it pays while the march's chain of planes takes longer
 // than that: up to some number of field values per sweep, more in FP32, whose

@@ -287,7 +287,9 @@ class Simulation:
 
     def tune_get(self):
         """{kind name: (variant, zchunk, waves, rows per wave)} for the stage
-        kinds and the fused stage pairs"""
+        kinds and the fused stage pairs; a stage kind in the automatic
+        configuration has zchunk -1 (a march) or -2 or -4 (bricks of so many
+        planes)"""
         out = {}
         for nm in _lib.STAGE_KINDS + _lib.PAIR_KINDS:
             k = _lib.KIND_NAMES.index(nm)

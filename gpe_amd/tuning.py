@@ -1,7 +1,8 @@
 """Persisted launch configurations of the stage kernels.
 
-The autotuner (gpe_autotune in the C ABI) times every compiled tile variant
-and several z-chunk lengths per stage kind on the resident field.  Results
+The autotuner (gpe_autotune in the C ABI) times the automatic choice and every
+compiled tile variant with several z-chunk lengths per stage kind on the
+resident field.  Results
 are kept in a JSON file keyed by (grid, order, precision, scheme, boundary
 condition, fusion) so a later run of the same problem skips the search; the
 library's gpe_tune_load applies an entry to a context (also from C and from
@@ -46,9 +47,10 @@ def apply(sim, path=DEFAULT_PATH):
 
 
 def tune(sim, reps=3, path=DEFAULT_PATH, store=True):
-    """Autotune sim's stage kernels (state unchanged) and persist the result."""
+    """Autotune sim's stage kernels (state unchanged) and persist the result.
+    Kinds that are left automatic (zchunk < 0) have no place in the entry."""
     got = sim.autotune(reps)
-    ent = {k: [v[0], v[1]] for k, v in got.items()}
+    ent = {k: [v[0], v[1]] for k, v in got.items() if v[1] >= 0}
     if store:
         table = load(path)
         table[sim.tune_key()] = ent

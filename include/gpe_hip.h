@@ -267,9 +267,13 @@ int gpe_energy_noalloc(const gpe_params *params, const void *psi, double *energy
 /* Launch configuration of the stage kernels.  Each stage kind (0 .. 14)
  * and each fused stage pair (16 .. 20; see gpe_prof_query for names) runs
  * with one of several compiled tile variants (waves x rows per wave) and a
- * z-chunk length (0 = automatic); a pair with variant -1 runs as its two
- * stages.  No reference counterpart: the reference has no device kernels to
- * configure. */
+ * z-chunk length (0: of a length chosen for the tile and grid); a pair with
+ * variant -1 runs as its two stages.  Every stage kind starts in the automatic
+ * configuration, where the library chooses the sweep for the kind and grid:
+ * short bricks, or a march with a tile and chunk of its choice.  Its zchunk is
+ * negative: -1 (and what gpe_tune_get gives, -2 and -4) sets it again, with any
+ * variant the kind may run.  No reference counterpart: the reference has no
+ * device kernels to configure. */
 int gpe_tune_set(gpe_ctx *ctx, int32_t kind, int32_t variant, int32_t zchunk);
 /* Fuse consecutive RK4 / Cash-Karp stages pairwise into one sweep each
  * (RK4: 7 field passes per step instead of 13; Cash-Karp: 14 per attempt
@@ -279,6 +283,10 @@ int gpe_tune_set(gpe_ctx *ctx, int32_t kind, int32_t variant, int32_t zchunk);
  * GPE_FP64 has no fused kernels: enable = 1 on a GPE_FP64 context returns
  * GPE_EINVAL. */
 int gpe_set_fusion(gpe_ctx *ctx, int32_t enable);
+/* The configuration as it was set or, for a stage kind in the automatic one, as
+ * it is chosen: zchunk -1 is a march with this variant, -2 and -4 are bricks of
+ * so many planes (variant: that of the march on larger grids).  waves and
+ * rows_per_wave are those of the kernel that runs. */
 int gpe_tune_get(gpe_ctx *ctx, int32_t kind, int32_t *variant, int32_t *zchunk, int32_t *waves,
                  int32_t *rows_per_wave);
 /* Stored launch configurations.  The autotuner's picks are kept in a JSON
@@ -296,10 +304,11 @@ int gpe_tune_get(gpe_ctx *ctx, int32_t kind, int32_t *variant, int32_t *zchunk, 
  * do not depend on the launch configuration.  No reference counterpart. */
 int gpe_tune_key(gpe_ctx *ctx, char *buf, int64_t cap);
 int gpe_tune_load(gpe_ctx *ctx, const char *path, int32_t *applied);
-/* Time every variant and several z-chunks of each stage kind (and, with
- * fusion on, of each stage pair) of the context's scheme on the resident
- * field (reps launches each) and keep the fastest; a pair runs fused only
- * where that beats its two stages.  The state is unchanged. */
+/* Time the automatic configuration and every variant with several z-chunks of
+ * each stage kind (and, with fusion on, of each stage pair) of the context's
+ * scheme on the resident field (reps launches each) and keep the fastest; a
+ * pair runs fused only where that beats its two stages.  The state is
+ * unchanged. */
 int gpe_autotune(gpe_ctx *ctx, int32_t reps);
 
 /* Kernel timing with HIP events recorded on the context's stream around
