@@ -181,8 +181,9 @@ class Batch:
         return v.value, z.value
 
     def autotune(self, reps=3):
-        """Pick tile variant and z-chunk per stage kind by timing the
-        batched launches on the current instances; commits no step."""
+        """Pick the automatic sweep or a tile variant and z-chunk per stage
+        kind by timing the batched launches on the current instances; commits
+        no step."""
         _lib.check(self._L.gpe_batch_autotune(self._b, int(reps)))
 
     # -- checkpoint / restart ------------------------------------------------

@@ -34,7 +34,8 @@ using namespace gpe;
 namespace {
 
 constexpr int kBatchDefaultVid = 0;
-// the default tile variant of stage kind k in a group of precision prec
+// the tile variant and chunk of stage kind k in a group of precision prec that
+// has more work than any rule below asks for
 int default_vid(int prec, int k) { return variant_allowed(prec == GPE_FP64, k, kBatchDefaultVid) ? kBatchDefaultVid : kVidF64Ck; }
 constexpr int kDefaultZc = 32;
 constexpr int kMaxGrid = 2048;  // persistent workgroups per batched launch
@@ -186,7 +187,7 @@ int group_of(gpe_batch *b, int prec, int order, int scheme) {
   scheme_kinds(scheme, &G.k0, &G.nk);
   for (int k = 0; k < K_COUNT; ++k) {
     G.vid[k] = default_vid(prec, k);
-    G.zc[k] = kDefaultZc;
+    G.zc[k] = kAutoChunk;
   }
   for (int q = 0; q < P_COUNT; ++q) {
     G.pfuse[q] = false;
@@ -322,8 +323,9 @@ StageArgs inst_args(const Inst &I, int kind, const gpe_step_state &st) {
   return A;
 }
 
-// How kind k of a group is swept.  A configuration that was set (by hand or by
-// the autotuner) stays; the default one is chosen here.
+// How kind k of a group whose grids have `sites` sites is swept.  A
+// configuration that was set (by hand or by the autotuner) stays; the automatic
+// one is chosen here.
 //
 // The group's sites together decide whether the chip is short of work: then
 // the chain of planes a workgroup marches through sets the time, and bricks or
@@ -351,9 +353,9 @@ StageArgs inst_args(const Inst &I, int kind, const gpe_step_state &st) {
 // All together, a whole iteration before and after: one 64^3 grid, FP32C RK4,
 // 292 -> 35 us; 6 grids of 48..128, FP64 RK4, 656 -> 359; 24 grids of 32..128,
 // FP32C RK4, 650 -> 596, FP64 RK45 3400 -> 2740.
-GroupSweep sweep_of(const Group &G, int k) {
+GroupSweep sweep_of(const Group &G, int k, long long sites) {
   const bool fp64 = G.prec == GPE_FP64;
-  if (G.vid[k] != default_vid(G.prec, k) || G.zc[k] != kDefaultZc) return {0, G.vid[k], G.zc[k], false};
+  if (G.zc[k] != kAutoChunk) return {0, G.vid[k], G.zc[k], false};
   if (k == G.k0 + G.nk - 1) {
     if (k == K_RK2_2 || (fp64 && k == K_EULER)) return {0, 3, 16, true};
     if (!fp64) return {0, k == K_EULER ? 1 : 4, 16, true};
@@ -361,12 +363,12 @@ GroupSweep sweep_of(const Group &G, int k) {
   }
   const int reads = stage_reads(k);
   if (!fp64) {
-    if (G.sites * reads <= 16000000) return {2, 0, 0, false};
-    return {0, reads == 1 ? 0 : G.sites <= 12000000 ? 4 : 1, 16, false};
+    if (sites * reads <= 16000000) return {2, 0, 0, false};
+    return {0, reads == 1 ? 0 : sites <= 12000000 ? 4 : 1, 16, false};
   }
-  if (reads == 1 && G.sites <= 10000000) return {4, 0, 0, false};
-  if (G.sites * reads <= 5000000) return {2, 0, 0, false};
-  if (G.sites <= 8000000) return {0, reads <= 4 ? 3 : 4, 16, false};
+  if (reads == 1 && sites <= 10000000) return {4, 0, 0, false};
+  if (sites * reads <= 5000000) return {2, 0, 0, false};
+  if (sites <= 8000000) return {0, reads <= 4 ? 3 : 4, 16, false};
   if (k == K_RK4_2 || reads >= 4) return {0, default_vid(G.prec, k), kDefaultZc, false};
   return {0, 3, 16, false};
 }
@@ -458,6 +460,15 @@ int ensure_partials(gpe_batch *b, int need) {
   return GPE_OK;
 }
 
+// Sites of a group's instances.
+long long sites_of(const gpe_batch *b, int group) {
+  long long n = 0;
+  for (int s = 0; s < b->cap; ++s)
+    if (b->slot[s].id >= 0 && b->slot[s].group == group)
+      n += (long long)b->slot[s].P.nx * b->slot[s].P.ny * b->slot[s].P.nz;
+  return n;
+}
+
 // Regenerate every group's work tables and partial ranges.  Stream idle.
 int rebuild(gpe_batch *b) {
   int rc;
@@ -467,13 +478,12 @@ int rebuild(gpe_batch *b) {
     G.slots.clear();
     for (int s = 0; s < b->cap; ++s)
       if (b->slot[s].id >= 0 && b->slot[s].group == (int)(&G - &b->groups[0])) G.slots.push_back(s);
-    G.sites = 0;
-    for (int s : G.slots) G.sites += (long long)b->slot[s].P.nx * b->slot[s].P.ny * b->slot[s].P.nz;
+    G.sites = sites_of(b, (int)(&G - &b->groups[0]));
     G.part_off = part;
     for (const Unit &u : units_of(G)) {
       int TX, TY;
       KindTable &T = u.pair >= 0 ? G.ptab[u.pair] : G.tab[u.kind];
-      const GroupSweep w = u.pair >= 0 ? GroupSweep{0, 0, G.pzc[u.pair], false} : sweep_of(G, u.kind);
+      const GroupSweep w = u.pair >= 0 ? GroupSweep{0, 0, G.pzc[u.pair], false} : sweep_of(G, u.kind, G.sites);
       if (u.pair >= 0)
         pair_tiles(G, G.pvid[u.pair], &TX, &TY);
       else
@@ -536,7 +546,7 @@ int enqueue_iteration(gpe_batch *b, bool fork) {
         L.pn = u.final_ ? b->d_pn : nullptr;
         L.pe = u.final_ ? b->d_pe : nullptr;
         L.grid = T.grid;
-        e = launch_sweep(G, k, sweep_of(G, k), L, s);
+        e = launch_sweep(G, k, sweep_of(G, k, G.sites), L, s);
       }
       if (e != hipSuccess) return fail(GPE_EHIP, "batched stage launch: %s", hipGetErrorString(e));
     }
@@ -936,7 +946,8 @@ int gpe_batch_tune_set(gpe_batch *b, int32_t precision, int32_t order, int32_t s
                        int32_t variant, int32_t zchunk) {
   if (!b) return fail(GPE_EINVAL, "batch is NULL");
   if (kind < 16 && (variant < 0 || variant >= N_TILE_VARIANTS)) return fail(GPE_EINVAL, "variant out of range");
-  if (zchunk < 0 || (zchunk > 0 && zchunk < 8)) return fail(GPE_EINVAL, "zchunk must be 0 or >= 8");
+  const bool automatic = kind < 16 && automatic_chunk(zchunk);
+  if (!automatic && (zchunk < 0 || (zchunk > 0 && zchunk < 8))) return fail(GPE_EINVAL, "zchunk must be 0 or >= 8");
   if ((precision != GPE_FP64 && precision != GPE_FP32C) || (order != 2 && order != 4))
     return fail(GPE_EINVAL, "bad precision or order");
   GPE_HIPCHK(hipStreamSynchronize(b->stream));
@@ -958,7 +969,7 @@ int gpe_batch_tune_set(gpe_batch *b, int32_t precision, int32_t order, int32_t s
   if (!variant_allowed(precision == GPE_FP64, kind, variant))
     return fail(GPE_EINVAL, "FP64 Cash-Karp stages do not run tile variant %d", variant);
   G.vid[kind] = variant;
-  G.zc[kind] = zchunk;
+  G.zc[kind] = automatic ? kAutoChunk : zchunk;
   b->dirty = true;
   return GPE_OK;
 }
@@ -975,19 +986,23 @@ int gpe_batch_tune_get(gpe_batch *b, int32_t precision, int32_t order, int32_t s
         return GPE_OK;
       }
       if (kind < G.k0 || kind >= G.k0 + G.nk) return fail(GPE_EINVAL, "kind %d is not a stage of scheme %d", kind, scheme);
-      if (variant) *variant = G.vid[kind];
-      if (zchunk) *zchunk = G.zc[kind];
+      const long long sites = sites_of(b, (int)(&G - &b->groups[0]));
+      if (G.zc[kind] == kAutoChunk && !sites) break;
+      const GroupSweep w = sweep_of(G, kind, sites);
+      if (variant) *variant = w.planes ? default_vid(precision, kind) : w.vid;
+      if (zchunk) *zchunk = w.planes ? -w.planes : G.zc[kind];
       return GPE_OK;
     }
+  // nothing set and nothing to choose for
   if (variant) *variant = kind >= 16 ? -1 : default_vid(precision, kind);
   if (zchunk) *zchunk = kind >= 16 ? 0 : kDefaultZc;
   return GPE_OK;
 }
 
-// Time every tile variant and z-chunk for each stage kind of every group
-// over the current instances (reps launches each, stage kernels only: the
-// control kernel does not run, so no state is committed) and keep the
-// fastest (the default configuration is timed as sweep_of sweeps it).
+// Time the automatic sweep and every tile variant and z-chunk for each stage
+// kind of every group over the current instances (reps launches each, stage
+// kernels only: the control kernel does not run, so no state is committed) and
+// keep the fastest.
 int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
   if (!b) return fail(GPE_EINVAL, "batch is NULL");
   if (reps < 1) reps = 1;
@@ -1008,41 +1023,43 @@ int gpe_batch_autotune(gpe_batch *b, int32_t reps) {
       const int v0 = G.vid[k], z0 = G.zc[k];
       int bv = v0, bz = z0;
       KindTable T;
+      std::vector<std::pair<int, int>> trials = {{v0, kAutoChunk}};
       for (int v = 0; v < N_TILE_VARIANTS; ++v)
-        for (int z : zcs) {
-          if (!variant_allowed(G.prec == GPE_FP64, k, v)) continue;
-          int TX, TY;
-          G.vid[k] = v;
-          G.zc[k] = z;
-          const GroupSweep w = sweep_of(G, k);
-          kind_tiles(w, &TX, &TY);
-          make_table(b, G, TX, TY, w, T.h, nullptr, 0);
-          if ((rc = upload_table(T)) || (rc = ensure_partials(b, T.n))) break;
-          BatchLaunch L;
-          L.insts = b->d_args + (size_t)k * b->cap;
-          L.work = T.d;
-          L.nwork = T.n;
-          L.active = b->d_active;
-          L.pn = fin ? b->d_pn : nullptr;
-          L.pe = fin ? b->d_pe : nullptr;
-          L.grid = T.grid;
-          hipError_t e = launch_sweep(G, k, w, L, b->stream);  // warm
-          e = e != hipSuccess ? e : hipEventRecord(e0, b->stream);
-          for (int r = 0; r < reps && e == hipSuccess; ++r) e = launch_sweep(G, k, w, L, b->stream);
-          e = e != hipSuccess ? e : hipEventRecord(e1, b->stream);
-          e = e != hipSuccess ? e : hipEventSynchronize(e1);
-          if (e != hipSuccess) {
-            rc = fail(GPE_EHIP, "autotune launch: %s", hipGetErrorString(e));
-            break;
-          }
-          float ms = 0.f;
-          (void)hipEventElapsedTime(&ms, e0, e1);
-          if (ms < best) {
-            best = ms;
-            bv = v;
-            bz = z;
-          }
+        for (int z : zcs)
+          if (variant_allowed(G.prec == GPE_FP64, k, v)) trials.push_back({v, z});
+      for (const auto &[v, z] : trials) {
+        int TX, TY;
+        G.vid[k] = v;
+        G.zc[k] = z;
+        const GroupSweep w = sweep_of(G, k, G.sites);
+        kind_tiles(w, &TX, &TY);
+        make_table(b, G, TX, TY, w, T.h, nullptr, 0);
+        if ((rc = upload_table(T)) || (rc = ensure_partials(b, T.n))) break;
+        BatchLaunch L;
+        L.insts = b->d_args + (size_t)k * b->cap;
+        L.work = T.d;
+        L.nwork = T.n;
+        L.active = b->d_active;
+        L.pn = fin ? b->d_pn : nullptr;
+        L.pe = fin ? b->d_pe : nullptr;
+        L.grid = T.grid;
+        hipError_t e = launch_sweep(G, k, w, L, b->stream);  // warm
+        e = e != hipSuccess ? e : hipEventRecord(e0, b->stream);
+        for (int r = 0; r < reps && e == hipSuccess; ++r) e = launch_sweep(G, k, w, L, b->stream);
+        e = e != hipSuccess ? e : hipEventRecord(e1, b->stream);
+        e = e != hipSuccess ? e : hipEventSynchronize(e1);
+        if (e != hipSuccess) {
+          rc = fail(GPE_EHIP, "autotune launch: %s", hipGetErrorString(e));
+          break;
         }
+        float ms = 0.f;
+        (void)hipEventElapsedTime(&ms, e0, e1);
+        if (ms < best) {
+          best = ms;
+          bv = v;
+          bz = z;
+        }
+      }
       if (T.d) (void)hipFree(T.d);
       G.vid[k] = rc ? v0 : bv;
       G.zc[k] = rc ? z0 : bz;

@@ -381,13 +381,17 @@ int gpe_batch_stats(gpe_batch *b, int32_t *instances, int32_t *running, int64_t 
 int gpe_batch_use_graph(gpe_batch *b, int32_t enable);
 /* Tile variant and z-chunk (0 = whole column) of one stage kind (0 .. 14)
  * or fused stage pair (16 .. 20, variant -1 = run as its two stages) for
- * the instances of (precision, order, scheme). */
+ * the instances of (precision, order, scheme).  A negative zchunk stands for a
+ * stage kind's automatic configuration, in which it starts, as for gpe_tune_set
+ * and gpe_tune_get: the sweep is chosen for the resident instances, and one
+ * that was read sets it again.  Where nothing is resident and nothing was set,
+ * gpe_batch_tune_get gives the tile and chunk of a large group. */
 int gpe_batch_tune_set(gpe_batch *b, int32_t precision, int32_t order, int32_t scheme, int32_t kind,
                        int32_t variant, int32_t zchunk);
 int gpe_batch_tune_get(gpe_batch *b, int32_t precision, int32_t order, int32_t scheme, int32_t kind,
                        int32_t *variant, int32_t *zchunk);
-/* Time every variant and z-chunk of every stage kind and stage pair over
- * the current instances and keep the fastest (a pair runs fused only where
+/* Time the automatic configuration and every variant and z-chunk of every
+ * stage kind and stage pair over the current instances and keep the fastest (a pair runs fused only where
  * that beats its two stages).  Commits no step. */
 int gpe_batch_autotune(gpe_batch *b, int32_t reps);
 

@@ -87,3 +87,33 @@ def test_refused_pairs_stay_refused(gpu):
             with pytest.raises(_lib.GpeError):
                 sim.tune_set("ck_6", *pair)
         assert sim.tune_get() == before
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+@pytest.mark.parametrize("scheme", ["rk4", "rk45"])
+def test_batch(gpu, scheme, precision):
+    from gpe_amd.batch import Batch
+    cfg = _cfg((48, 40, 36), scheme=scheme, precision=precision)
+    psi = ic.vortex_ring(cfg, 2.0)
+    kinds = KINDS[scheme]
+    print("[case] batch readings", scheme, precision, flush=True)
+
+    def run(setting):
+        with Batch() as b:
+            i = b.add(cfg, psi, 2)
+            auto = [b.tune_get(precision, 4, scheme, k) for k in kinds]
+            assert all(z < 0 for _, z in auto)
+            for k, a in zip(kinds, auto):
+                v = 4 if precision == "fp64" and scheme == "rk45" else 0
+                if setting == "default":
+                    b.tune_set(precision, 4, scheme, k, v, 32)
+                    assert b.tune_get(precision, 4, scheme, k) == (v, 32)
+                elif setting == "restored":
+                    b.tune_set(precision, 4, scheme, k, 3, 16)
+                    b.tune_set(precision, 4, scheme, k, *a)
+                    assert b.tune_get(precision, 4, scheme, k) == a
+            b.run_to_completion(chunk=2)
+            return b.download(i)
+
+    want = run("automatic")
+    assert np.array_equal(run("default"), want) and np.array_equal(run("restored"), want)
