@@ -249,11 +249,10 @@ struct HostField {
   }
 };
 
-// Move `bytes` of a field through the staging buffers.  bus(buf, at, len) puts
-// the device work of bytes [at, at + len) on the stage's stream.
+// Move `bytes` of a field through the reserved staging buffers.  bus(buf, at,
+// len) puts the device work of bytes [at, at + len) on the stage's stream.
 template <typename Bus>
 int through(Stage &st, const HostField &h, size_t bytes, bool out, Bus bus) {
-  if (!st.reserve(bytes)) return fail(GPE_ENOMEM, "staging buffers");
   const size_t n = (bytes + kChunk - 1) / kChunk;
   auto put = [&](size_t i) {
     const size_t at = i * kChunk;
@@ -280,6 +279,81 @@ int through(Stage &st, const HostField &h, size_t bytes, bool out, Bus bus) {
     return fail(GPE_EHIP, "field transfer: %s", hipGetErrorString(e));
   }
   return GPE_OK;
+}
+
+// ---- without page-locked memory ----------------------------------------------
+// Where none is to be had (a limit on locked pages, a host short of memory), a
+// field moves by synchronous copies of the caller's pages, converted here in
+// pieces of kPlainWords.
+constexpr size_t kPlainWords = (size_t)1 << 18;
+
+int plain_upload(const HostField &h, size_t bytes, bool split, void *hi, void *lo) {
+  constexpr size_t word = 8;  // of a value that is split
+  const size_t piece = split ? kPlainWords * word : h.plane == h.pitch ? bytes : h.plane;
+  std::vector<double> v;
+  std::vector<float> w;
+  if (split) {
+    v.resize(kPlainWords);
+    w.resize(2 * kPlainWords);
+  }
+  for (size_t at = 0; at < bytes; at += piece) {
+    const size_t len = std::min(piece, bytes - at);
+    if (!split) {
+      const size_t k = at / h.plane;
+      GPE_HIPCHK(hipMemcpy((char *)hi + at, h.base + k * h.pitch, len, hipMemcpyHostToDevice));
+      continue;
+    }
+    const size_t n = len / word;
+    h.piece((char *)v.data(), at, len, false);
+    float *whi = w.data(), *wlo = whi + kPlainWords;
+    for (size_t i = 0; i < n; ++i) {
+      whi[i] = (float)v[i];
+      wlo[i] = (float)(v[i] - (double)whi[i]);
+    }
+    GPE_HIPCHK(hipMemcpy((float *)hi + at / word, whi, n * 4, hipMemcpyHostToDevice));
+    if (lo) GPE_HIPCHK(hipMemcpy((float *)lo + at / word, wlo, n * 4, hipMemcpyHostToDevice));
+  }
+  if (lo && !split) {
+    GPE_HIPCHK(hipMemset(lo, 0, bytes));
+    GPE_HIPCHK(hipStreamSynchronize(nullptr));
+  }
+  return GPE_OK;
+}
+
+// stored: bytes of a stored word (hi's; lo: the compensated form's, or null);
+// word: of a host word.
+int plain_download(size_t stored, size_t word, size_t words, const void *hi, const void *lo, void *dst) {
+  if (stored == word && !lo) {
+    GPE_HIPCHK(hipMemcpy(dst, hi, words * word, hipMemcpyDeviceToHost));
+    return GPE_OK;
+  }
+  std::vector<double> v(kPlainWords);
+  std::vector<float> w(kPlainWords), l(kPlainWords, 0.0f);
+  for (size_t at = 0; at < words; at += kPlainWords) {
+    const size_t n = std::min(kPlainWords, words - at);
+    if (stored == 8) {
+      GPE_HIPCHK(hipMemcpy(v.data(), (const double *)hi + at, n * 8, hipMemcpyDeviceToHost));
+    } else {
+      GPE_HIPCHK(hipMemcpy(w.data(), (const float *)hi + at, n * 4, hipMemcpyDeviceToHost));
+      if (lo) GPE_HIPCHK(hipMemcpy(l.data(), (const float *)lo + at, n * 4, hipMemcpyDeviceToHost));
+      for (size_t i = 0; i < n; ++i) v[i] = (double)w[i] + (double)l[i];
+    }
+    if (word == 8)
+      std::memcpy((double *)dst + at, v.data(), n * 8);
+    else
+      for (size_t i = 0; i < n; ++i) ((float *)dst)[at + i] = (float)v[i];
+  }
+  return GPE_OK;
+}
+
+template <typename F>
+int plainly(F f) {
+  (void)hipGetLastError();  // the refusal is not the next launch's error
+  try {
+    return f();
+  } catch (const std::bad_alloc &) {
+    return fail(GPE_ENOMEM, "host memory of a field transfer");
+  }
 }
 
 // A conversion kernel over n words on the stage's stream.
@@ -323,10 +397,11 @@ int field_upload(int prec, size_t plane, int nz, const void *src, int host_type,
     return fail(GPE_EINVAL, "FP64 storage takes complex128 host data");
   const size_t esz = host_type == GPE_HOST_C128 ? 16 : 8, bytes = plane * (size_t)nz * esz;
   const bool comp = prec == GPE_FP32C, split = prec != GPE_FP64 && host_type == GPE_HOST_C128;
-  Lease lease;
-  if (!lease.st) return fail(GPE_ENOMEM, "staging buffers");
-  Stage &st = *lease.st;
   const HostField h{(char *)const_cast<void *>(src) + row_off * esz, plane * esz, src_pitch_planes * esz};
+  Lease lease;
+  if (!lease.st || !lease.st->reserve(bytes))
+    return plainly([&] { return plain_upload(h, bytes, split, hi, comp ? lo : nullptr); });
+  Stage &st = *lease.st;
   if (comp && !split) {
     const size_t n = 2 * plane * (size_t)nz;
     GPE_HIPCHK(launch(st, n, fill_zero, (float *)lo));
@@ -352,7 +427,8 @@ int field_download(int prec, size_t plane, int nz, const void *hi, const void *l
 int words_download(int stored, size_t sites, const void *hi, const void *lo, void *dst, int host_type) {
   const size_t esz = host_type == GPE_HOST_C128 ? 16 : 8, bytes = sites * esz;
   Lease lease;
-  if (!lease.st) return fail(GPE_ENOMEM, "staging buffers");
+  if (!lease.st || !lease.st->reserve(bytes))
+    return plainly([&] { return plain_download(stored / 2, esz / 2, 2 * sites, hi, lo, dst); });
   Stage &st = *lease.st;
   const HostField h{(char *)dst, bytes, bytes};
   return through(st, h, bytes, true, [&](char *buf, size_t at, size_t len) -> hipError_t {
