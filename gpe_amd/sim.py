@@ -197,14 +197,21 @@ class Simulation:
         w = _lib.ZERO_FILES[which]
         n = ctypes.c_int64()
         # room for a dense tangle's points (memory that is not written costs
-        # nothing); more than that are counted first and fetched again
+        # nothing, and the rest is given back); more than that, or more than
+        # there is room for, are counted first and fetched again
         cap = max(1024, self.cfg.nx * self.cfg.ny * self.cfg.nz // 16)
-        while True:
+        try:
             out = np.empty(cap, dtype=_lib.ZERO_DTYPE)
-            _lib.check(self._L.gpe_sim_zeros(self._ctx, w, out.ctypes.data_as(ctypes.c_void_p), cap, ctypes.byref(n)))
-            if n.value <= cap:
-                return out[:n.value]
+        except MemoryError:
+            cap, out = 0, None
+        while True:
+            buf = None if out is None else out.ctypes.data_as(ctypes.c_void_p)
+            _lib.check(self._L.gpe_sim_zeros(self._ctx, w, buf, cap, ctypes.byref(n)))
+            if out is not None and n.value <= cap:
+                out.resize(n.value, refcheck=False)
+                return out
             cap = n.value
+            out = np.empty(cap, dtype=_lib.ZERO_DTYPE)
 
     def save_zeros(self, proc_dir):
         """zeros<p>.dat, re_zeros<p>.dat and im_zeros<p>.dat of the resident
