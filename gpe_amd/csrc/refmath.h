@@ -27,8 +27,13 @@
 //
 // Both are built from IEEE double +, -, *, /, sqrt, fma, ldexp, frexp and
 // rint, which round (or are exact) identically on the host and the device,
-// so a host build of this header gives the device's bits.  Callers compile
-// it with -ffp-contract=off (no contraction the host build would not do).
+// so a host build of this header gives the device's bits; but for hypot in
+// its inner range, where the device takes hypot_fast (from the hardware's
+// approximate reciprocal square root): the GPU test of this header compares
+// 2 million arguments in each of 21 classes, dense at the limits of that range
+// and where the formulas meet, with the host libm: equal in every bit.
+// Callers compile it with -ffp-contract=off (no contraction the host build
+// would not do).
 #pragma once
 #include <cmath>
 

@@ -3,9 +3,10 @@
 hypot_ref must equal the host libm's hypot (the reference's abs of a
 complex) in every bit; pow_cr must be the correctly rounded x**y (checked
 against 60-digit decimal arithmetic) and equal the host libm's pow on all
-but a small fraction of the step control's arguments.  The header uses only
-operations that round identically on the host and the device, so these
-host results are the device's."""
+but a small fraction of the step control's arguments.  pow_cr uses only
+operations that round identically on the host and the device, so its host
+results are the device's; the device's hypot_ref has a fast inner range of its
+own, compared with the host libm by test_hypot_gpu.py."""
 import ctypes
 import os
 import subprocess
