@@ -81,3 +81,26 @@ def test_norm_history_equals_single_steps(gpu, scheme):
         last = sim.norm()
     assert np.array_equal(together, single)
     assert abs(single[-1] - last) <= 1e-13 * last
+
+
+@pytest.mark.parametrize("shape", [(5, 5, 5), (64, 8, 6), (65, 9, 7), (63, 17, 31), (130, 24, 5)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "fp32c"])
+def test_brick_energy_equals_march(gpu, shape, precision):
+    # every site's term has the same bits either way and they are summed in
+    # double: the sums differ by at most (terms) 2^-53 of the sum of |term|
+    from gpe_amd.sim import Simulation
+    cfg = _cfg(shape, precision=precision, scheme="euler", order=2, bcs=1)
+    psi = _field(cfg)
+    print("[case] brick energy", shape, precision, flush=True)
+    got = []
+    for tile in (None, (4, 8), (0, 8)):
+        with Simulation(cfg, psi, tuned=False) as sim:
+            if tile:
+                sim.tune_set("energy", *tile)
+            got.append(sim.energy())
+    lap = sum((np.roll(psi, 1, a) - 2 * psi + np.roll(psi, -1, a)) / d ** 2
+              for a, d in ((0, cfg.dz), (1, cfg.dy), (2, cfg.dx)))
+    m = np.abs(psi)
+    terms = 1.01 * np.sum(np.abs(lap).astype(np.float64) * m + 0.5 * m.astype(np.float64) ** 4) * cfg.dx * cfg.dy * cfg.dz
+    for g in got[1:]:
+        assert abs(g - got[0]) <= psi.size * 2.0 ** -53 * terms
