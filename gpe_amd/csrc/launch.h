@@ -23,8 +23,9 @@ constexpr Tile kTiles[N_TILE_VARIANTS] = {{4, 4}, {8, 2}, {16, 1}, {4, 2}, {8, 1
 // 4th-order last-stage instantiation is allocated the full 256 VGPRs and
 // still spills to scratch (484 and 292 B per lane in the single-simulation
 // kernel, 624 and 372 B batched); (16,1) spills too, but under a 128-VGPR
-// budget, and passes.  The FP64 Cash-Karp default is (8,1), which needs no
-// scratch in any stage.
+// budget, and passes.  (8,1) needs no scratch in any stage; the automatic
+// march takes it for the last stage, but (16,1) for two of the others in 4th
+// order (march_vid).
 constexpr int kVidF64Ck = 4;
 constexpr bool variant_allowed(bool fp64, int kind, int vid) {
   return vid >= 0 && vid < N_TILE_VARIANTS && !(fp64 && kind >= K_CK_1 && kind <= K_CK_6 && vid <= 1);
@@ -130,7 +131,10 @@ inline int brick_planes(bool fp64, int kind, int radius, int nx, int ny, int nz)
 // plane, so the variants with the fewest registers per lane and more
 // workgroups win ((4,2) against (8,2), 4th order: 256^3 rk4_4 283 -> 229 us,
 // 512^3 rk4_3 1590 -> 1300, ck_2 against (8,1) 2060 -> 1340; (16,1) for ck_3
-// and ck_4, 256^3 319 -> 261); the FP32 ones keep (8,2) but for those that
+// and ck_4, 256^3 319 -> 261, though these two spill 36 and 84 B a lane in 4th
+// order: spilling is what the shapes that variant_allowed refuses had in
+// common, so test_march_gpu.py holds the automatic fields to (8,1)'s bit for
+// bit on either side of every line); the FP32 ones keep (8,2) but for those that
 // store little or read one field (rk4_1 at 256^3 82 -> 65, rk4_2 157 -> 118).
 inline int march_vid(bool fp64, int kind, int radius, long long n) {
   const bool r2 = radius == 2;
@@ -157,8 +161,12 @@ inline int march_vid(bool fp64, int kind, int radius, long long n) {
 // rounds of zc + 2R planes each, and the chunk with the smallest product wins:
 // long enough that few planes are read twice, and with no round that is nearly
 // empty (FP64 ck_6 at 192^3: chunks of 8, 16, 32, 64 planes take 7, 4, 2, 1
-// rounds and 250, 243, 223, 208 us).  Over grids of 0.5 .. 134 M sites, every
-// kind and tile, it comes within 1 .. 2 % of the best of 8, 16, 32 and 64.
+// rounds and 250, 243, 223, 208 us).  Against the best of chunks of 8, 16, 32
+// and 64 in the same tile (261 kinds: seven grids of 2 .. 134 M sites, FP64 and
+// FP32C, both orders, every scheme) it takes 0.99 times as long in the mean, 1.00
+// in the median, 0.77 .. 1.14 at the ends and at most 1.045 in nine of ten; the
+// worst are FP64 kinds in the small (4,2) tile (256^3 rk4_1 159 us against 139
+// in chunks of 32).
 constexpr int kCUs = 256;
 inline int march_chunk(int nx, int ny, int nz, int vid, int radius, int resident) {
   const Tile t = kTiles[vid];
