@@ -197,8 +197,10 @@ class Simulation:
         w = _lib.ZERO_FILES[which]
         n = ctypes.c_int64()
         # room for a dense tangle's points (memory that is not written costs
-        # nothing, and the rest is given back); more than that, or more than
-        # there is room for, are counted first and fetched again
+        # nothing, and a rest of more than 64 MiB of address space is given
+        # back; cutting a smaller one takes up to 30 us of some 400 at 256^3);
+        # more points than that, or than there is room for, are counted first
+        # and fetched again
         cap = max(1024, self.cfg.nx * self.cfg.ny * self.cfg.nz // 16)
         try:
             out = np.empty(cap, dtype=_lib.ZERO_DTYPE)
@@ -208,8 +210,9 @@ class Simulation:
             buf = None if out is None else out.ctypes.data_as(ctypes.c_void_p)
             _lib.check(self._L.gpe_sim_zeros(self._ctx, w, buf, cap, ctypes.byref(n)))
             if out is not None and n.value <= cap:
-                out.resize(n.value, refcheck=False)
-                return out
+                if (cap - n.value) * out.itemsize > 64 << 20:
+                    out.resize(n.value, refcheck=False)
+                return out[:n.value]
             cap = n.value
             out = np.empty(cap, dtype=_lib.ZERO_DTYPE)
 

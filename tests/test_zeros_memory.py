@@ -1,5 +1,6 @@
-"""Memory of Simulation.zeros, without a GPU: the result holds its points and
-no more, and a grid whose dense list would not fit memory is counted first."""
+"""Memory of Simulation.zeros, without a GPU: the result holds its points and at
+most 64 MiB more, and a grid whose dense list would not fit memory is counted
+first."""
 import ctypes
 
 import numpy as np
@@ -33,12 +34,13 @@ def _sim(count, n=64):
     return sim
 
 
+@pytest.mark.parametrize("n", [64, 320, 512])
 @pytest.mark.parametrize("count", [0, 1, 1000, 16384, 16385, 40000])
-def test_result_holds_its_points_only(count):
-    got = _sim(count).zeros()
+def test_result_holds_its_points(count, n):
+    got = _sim(count, n).zeros()
     assert got.dtype == _lib.ZERO_DTYPE and np.array_equal(got["cell"], np.arange(count))
     held = got if got.base is None else got.base
-    assert held.nbytes <= max(count, 1) * _lib.ZERO_DTYPE.itemsize
+    assert held.nbytes <= got.nbytes + (64 << 20)
 
 
 def test_list_that_does_not_fit_is_counted_first(monkeypatch):
